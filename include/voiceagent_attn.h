@@ -291,8 +291,11 @@ typedef struct va_varlen_args {
    * slot_mapping[i] (slot < 0 skips), as store_kvcache would. */
   const void* slot_mapping;
   int32_t slot_dtype;
-  /* Unused (no varlen launch needs a workspace; va_varlen_workspace_bytes
-   * returns 0).  An FP8 pool's prefix rows are converted to the 16-bit type
+  /* Optional (no varlen launch needs a workspace; va_varlen_workspace_bytes
+   * returns 0): with at least va_varlen_split_workspace_bytes, 16-byte
+   * aligned, the launch may split long items' keys over several workgroups.
+   * No initialisation needed; launches sharing one must be ordered on one
+   * stream.  An FP8 pool's prefix rows are converted to the 16-bit type
    * (code * scale, rounded once) inside the kernel, tile by tile, and its
    * new rows are stored quantised after the attention. */
   void* workspace;
@@ -316,6 +319,13 @@ int va_varlen_attention(const va_varlen_args* args, void* stream);
 /* Bytes of workspace va_varlen_attention needs: always 0 (kept for callers
  * written against the earlier contract). */
 size_t va_varlen_workspace_bytes(const va_varlen_args* args);
+
+/* Bytes of workspace with which va_varlen_attention may split these
+ * arguments' long items over several workgroups (few items, or some with far
+ * more keys than the others); 0 where splitting cannot help.  Without it the
+ * launch gives the same result unsplit.  Depends on the current device's
+ * compute-unit count. */
+size_t va_varlen_split_workspace_bytes(const va_varlen_args* args);
 
 /* ----------------------------------------------------------------- misc */
 const char* va_last_error(void);

@@ -1,0 +1,116 @@
+"""Varlen launches whose long items are cut into pieces over several
+workgroups and merged (varlen_merge_kernel), at the sizes where the plan, the
+block-id windows (64 tiles of 64 keys) and the piece edges can go wrong:
+against the oracle (2e-2 for 16-bit inputs, the suite's bound) and against the
+same launch without a workspace, which runs unsplit.  Both forms keep fp32
+sums and differ in their order and in the reference maximum of P's 16-bit
+rounding, so they agree to two 16-bit output roundings and P's: 2^-7 of the
+largest |v| (under 5 for these N(0, 1) values)."""
+import math
+
+import pytest
+import torch
+
+from oracle import attention as oracle
+from voiceagent_amd import _native as N
+from voiceagent_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _cu(lens):
+    return torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).to(torch.int32)
+
+
+# (prefix, new tokens) per sequence
+CASES = {
+    "one_decode_past_the_id_window": [(64 * 64 + 5, 1)],
+    "window_edges": [(64 * 64, 3), (64 * 64 - 1, 1), (64 * 128, 70)],
+    "decodes_beside_prompts": [(n, 1) for n in (1, 15, 16, 17, 63, 64, 700, 2500, 4097)]
+                              + [(0, 300), (0, 1), (0, 65), (33, 130)],
+    "short_chunks_long_prefixes": [(3000, 8), (2049, 17), (1500, 64), (1, 2)],
+    "long_prompt": [(0, 1100)],
+    "with_empty_sequences": [(0, 0), (900, 1), (700, 0), (0, 270), (0, 0)],
+    "many_sequences": [(130 + 7 * i, 1 + i % 3) for i in range(60)],
+}
+
+
+@pytest.mark.parametrize("kv", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("hq,hkv,d,bs,i64,hnd", [(16, 8, 128, 16, False, False),
+                                                 (32, 4, 128, 48, True, True),
+                                                 (14, 14, 64, 8, False, False),
+                                                 (16, 2, 64, 16, True, False)])
+@pytest.mark.parametrize("name", list(CASES))
+def test_split_launch(dev, monkeypatch, name, hq, hkv, d, bs, i64, hnd, kv):
+    seqs = CASES[name]
+    gen = torch.Generator().manual_seed(len(name) + hq + d + bs)
+    dt = torch.float16 if kv == "f16" else torch.bfloat16
+    ql, kl = [n for _, n in seqs], [p + n for p, n in seqs]
+    need = [math.ceil(n / bs) for n in kl]
+    nb, width = sum(need) + 3, max(need)
+    perm = torch.randperm(nb, generator=gen).tolist()
+    table = torch.full((len(seqs), width), -1, dtype=torch.int64 if i64 else torch.int32)
+    at, slots = 0, []
+    for s, m in enumerate(need):
+        table[s, :m] = torch.tensor(perm[at:at + m])
+        at += m
+        slots += [int(table[s, j // bs]) * bs + j % bs for j in range(seqs[s][0], kl[s])]
+    slots = torch.tensor(slots, dtype=torch.int32)
+    shape = (nb, hkv, bs, d) if hnd else (nb, bs, hkv, d)
+    layout = ops.LAYOUT_HND if hnd else ops.LAYOUT_NHD
+    ks, vs = (0.05, 0.08) if kv == "fp8" else (1.0, 1.0)
+    kp, vp = (torch.randn(shape, generator=gen) for _ in range(2))
+    if kv == "fp8":
+        kp, vp = oracle.quantize_fp8(kp, ks), oracle.quantize_fp8(vp, vs)
+    else:
+        kp, vp = kp.to(dt), vp.to(dt)
+    q = torch.randn(sum(ql), hq, d, generator=gen).to(dt)
+    k, v = (torch.randn(sum(ql), hkv, d, generator=gen).to(dt) for _ in range(2))
+    cu_q, cu_k = _cu(ql), _cu(kl)
+    print(f"{name} {hq}/{hkv}x{d} block {bs} {kv}", flush=True)
+
+    def call():
+        kd, vd = kp.to(dev), vp.to(dev)
+        out = ops.varlen_attention(q.to(dev), k.to(dev), v.to(dev), cu_q.to(dev), cu_k.to(dev),
+                                   max(ql), max(kl), scale=d ** -0.5, causal=True, k_cache=kd,
+                                   v_cache=vd, block_tables=table.to(dev),
+                                   slot_mapping=slots.to(dev), layout=layout, k_scale=ks,
+                                   v_scale=vs)
+        torch.cuda.synchronize()
+        return out.float().cpu(), kd.cpu(), vd.cpu()
+
+    out, kd, vd = call()
+    ref = oracle.varlen_attention(q, k, v, cu_q, cu_k, d ** -0.5, True, k_cache=kp, v_cache=vp,
+                                  block_tables=table, layout=layout, k_scale=ks, v_scale=vs)
+    assert (out - ref).abs().max().item() <= 2e-2
+    ek, ev = oracle.store_kvcache(k, v, kp, vp, slots, layout=layout, k_scale=ks, v_scale=vs)
+    as_bytes = torch.uint8 if kv == "fp8" else torch.int16
+    assert torch.equal(kd.view(as_bytes), ek.view(as_bytes))
+    assert torch.equal(vd.view(as_bytes), ev.view(as_bytes))
+    # Without a workspace (the Python path, told that none helps): unsplit.
+    monkeypatch.setattr(ops, "_FAST_LOADED", True)
+    monkeypatch.setattr(ops, "_FAST", None)
+
+    real = N.lib()
+
+    class Unsplit:
+        def __getattr__(self, fn):
+            return (lambda args: 0) if fn == "va_varlen_split_workspace_bytes" else getattr(real, fn)
+
+    monkeypatch.setattr(N, "lib", Unsplit)
+    whole, _, _ = call()
+    assert (whole - out).abs().max().item() <= 5 * 2 ** -7
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(14, 14, 64), (16, 8, 128)])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("lens", [[700], [300, 1, 900, 64], [1, 2, 1300]])
+def test_split_launch_without_a_pool(dev, hq, hkv, d, causal, lens):
+    gen = torch.Generator().manual_seed(sum(lens) + d)
+    q = torch.randn(sum(lens), hq, d, generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn(sum(lens), hkv, d, generator=gen).to(torch.bfloat16) for _ in range(2))
+    cu = _cu(lens)
+    out = ops.varlen_attention(q.to(dev), k.to(dev), v.to(dev), cu.to(dev), cu.to(dev), max(lens),
+                               max(lens), scale=d ** -0.5, causal=causal)
+    ref = oracle.varlen_attention(q, k, v, cu, cu, d ** -0.5, causal)
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2

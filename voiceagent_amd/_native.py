@@ -201,6 +201,7 @@ SIGNATURES = {
     "va_paged_decode_noalloc": (c_int32, [ctypes.POINTER(DecodeArgs), c_void_p]),
     "va_varlen_attention": (c_int32, [ctypes.POINTER(VarlenArgs), c_void_p]),
     "va_varlen_workspace_bytes": (c_size_t, [ctypes.POINTER(VarlenArgs)]),
+    "va_varlen_split_workspace_bytes": (c_size_t, [ctypes.POINTER(VarlenArgs)]),
     "va_qk_norm_rope": (c_int32, [ctypes.POINTER(QkNormRopeArgs), c_void_p]),
     "va_last_error": (ctypes.c_char_p, []),
     "va_abi_version": (c_int32, []),

@@ -26,12 +26,14 @@ namespace {
 using DecodeFn = int (*)(const va_decode_args*, void*);
 using DecodeWsFn = size_t (*)(const va_decode_args*);
 using VarlenFn = int (*)(const va_varlen_args*, void*);
+using VarlenWsFn = size_t (*)(const va_varlen_args*);
 using StoreFn = int (*)(const va_store_args*, void*);
 using RopeFn = int (*)(const va_qk_norm_rope_args*, void*);
 
 DecodeFn g_decode = nullptr;
 DecodeWsFn g_decode_ws = nullptr;
 VarlenFn g_varlen = nullptr;
+VarlenWsFn g_varlen_ws = nullptr;
 StoreFn g_store = nullptr;
 RopeFn g_rope = nullptr;
 
@@ -103,11 +105,12 @@ bool index_vector(const at::Tensor& t, int64_t n) {
   return t.dim() == 1 && t.numel() >= n && t.is_contiguous() && index_code(t.scalar_type()) >= 0;
 }
 
-void set_entries(int64_t decode, int64_t decode_ws, int64_t varlen, int64_t store,
-                 int64_t rope) {
+void set_entries(int64_t decode, int64_t decode_ws, int64_t varlen, int64_t varlen_ws,
+                 int64_t store, int64_t rope) {
   g_decode = reinterpret_cast<DecodeFn>(static_cast<intptr_t>(decode));
   g_decode_ws = reinterpret_cast<DecodeWsFn>(static_cast<intptr_t>(decode_ws));
   g_varlen = reinterpret_cast<VarlenFn>(static_cast<intptr_t>(varlen));
+  g_varlen_ws = reinterpret_cast<VarlenWsFn>(static_cast<intptr_t>(varlen_ws));
   g_store = reinterpret_cast<StoreFn>(static_cast<intptr_t>(store));
   g_rope = reinterpret_cast<RopeFn>(static_cast<intptr_t>(rope));
 }
@@ -356,6 +359,16 @@ int64_t varlen_attention(const at::Tensor& q, const c10::optional<at::Tensor>& k
   a.max_seqlen_k = (int32_t)max_seqlen_k;
   a.causal = causal ? 1 : 0;
   a.scale = (float)scale;
+  // Memory for split items, of this call alone (the wrapper's rule: ops.py).
+  at::Tensor ws;
+  if (const size_t need = g_varlen_ws(&a)) {
+    try {
+      ws = at::empty({(int64_t)need}, q.options().dtype(at::kByte));
+      a.workspace = ws.data_ptr();
+      a.workspace_bytes = need;
+    } catch (const c10::OutOfMemoryError&) {
+    }
+  }
   return g_varlen(&a, reinterpret_cast<void*>(static_cast<intptr_t>(stream)));
 }
 

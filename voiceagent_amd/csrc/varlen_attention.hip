@@ -1,6 +1,8 @@
 // Host side of the varlen attention: argument checks and launch dispatch
 // (kernel in varlen_kernel.h, instantiated per element type and head_dim in
 // varlen_{bf16,f16}_d{64,128}.hip).
+#include <algorithm>
+
 #include "varlen_kernel.h"
 
 namespace va {
@@ -24,6 +26,62 @@ static int varlen_native(const va_varlen_args* a, void* stream);
 extern "C" size_t va_varlen_workspace_bytes(const va_varlen_args* a) {
   (void)a;
   return 0;
+}
+
+namespace va {
+
+// Workspace of a split launch: pieces' o, (m, l), heads and counts.
+struct SplitLayout {
+  size_t o, ml, head, count, total;
+};
+static SplitLayout split_layout(int head_dim) {
+  const size_t pieces = (size_t)kXcds * kSplitSlots;
+  SplitLayout l;
+  l.o = 0;
+  l.ml = l.o + pieces * kRowsPerWG * head_dim * sizeof(float);
+  l.head = l.ml + pieces * kRowsPerWG * sizeof(float2);
+  l.count = l.head + pieces * sizeof(int4);
+  l.total = l.count + 256;
+  return l;
+}
+
+// Whether a launch may gain from splitting its items, from what the host
+// knows.  The longest item may take as many tiles as the longest prompt or
+// the block table holds (the lengths themselves are on the device); with
+// items of half that on average, a slot's share is the piece the device would
+// choose.  The longest item has to exceed it by a quarter and five tiles
+// (~10 us): the pieces' partials and the merge launch cost about half that.
+// (9 prompts of 60-594 tokens and 24 decoding sequences beside three prompts
+// of 530, which this leaves whole, lost 2.5-3.4 us to a merge launch with
+// nothing to merge.)
+static bool split_wanted(const va_varlen_args* a) {
+  if (a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0) return false;
+  const int G = a->num_heads / a->num_kv_heads;
+  if (G != 1 && G != 2 && G != 4 && G != 8) return false;
+  if (a->head_dim != 64 && a->head_dim != 128) return false;
+  if (a->num_seqs <= 0 || a->total_q <= 0) return false;
+  const int BQ = kRowsPerWG / G;
+  if (!a->causal && a->pool.k == nullptr && a->max_seqlen_q <= BQ) return false;  // kOnce
+  const int64_t pairs = (int64_t)a->num_seqs * a->num_kv_heads;
+  if ((pairs + kXcds - 1) / kXcds > 64) return false;  // the plan holds a pair per lane
+  const int64_t table_keys =
+      a->pool.k != nullptr ? (int64_t)a->table_width * a->pool.block_size : 0;
+  const int64_t keys = a->max_seqlen_q > table_keys ? a->max_seqlen_q : table_keys;
+  const int64_t longest = (keys + kKeyTile - 1) / kKeyTile;
+  const int64_t slots = 2 * (int64_t)current_device_cus() / kXcds;  // of one XCD
+  const int64_t items =
+      (a->num_kv_heads * ((int64_t)a->total_q / BQ + a->num_seqs) + kXcds - 1) / kXcds;
+  const int64_t over = std::min<int64_t>(std::max(slots - items / 4, (slots + 1) / 2), kSplitSlots / 2);
+  const int64_t piece = std::max<int64_t>(items * longest / 2 / over, kSplitMinTiles);
+  return longest >= piece + piece / 4 + 5;
+}
+
+}  // namespace va
+
+extern "C" size_t va_varlen_split_workspace_bytes(const va_varlen_args* a) {
+  using namespace va;
+  if (a == nullptr || a->struct_size != sizeof(va_varlen_args)) return 0;
+  return split_wanted(a) ? split_layout(a->head_dim).total : 0;
 }
 
 extern "C" int va_varlen_attention(const va_varlen_args* a, void* stream) {
@@ -201,6 +259,26 @@ int va::varlen_native(const va_varlen_args* a, void* stream) {
   p.bs_div = make_fastdiv((uint32_t)p.block_size);
   p.hkv_div = make_fastdiv((uint32_t)a->num_kv_heads);
   p.slot_small = (int64_t)p.num_blocks * p.block_size <= ((int64_t)1 << 31);
+  // A tile's 16 rows of one block are copied from one base with 32-bit offsets.
+  p.block16 = has_pool && p.block_size % 16 == 0 && p.s_slot >= 0 &&
+              15 * p.s_slot + a->head_dim * kv_eb < ((int64_t)1 << 31);
+
+  p.split = 0;
+  p.part_o = nullptr;
+  p.part_ml = nullptr;
+  p.part_head = nullptr;
+  p.part_count = nullptr;
+  if (a->workspace != nullptr && (uintptr_t)a->workspace % 16 == 0 && split_wanted(a)) {
+    const SplitLayout l = split_layout(a->head_dim);
+    if (a->workspace_bytes >= l.total) {
+      char* const ws = (char*)a->workspace;
+      p.split = 1;
+      p.part_o = (float*)(ws + l.o);
+      p.part_ml = (float2*)(ws + l.ml);
+      p.part_head = (int4*)(ws + l.head);
+      p.part_count = (int32_t*)(ws + l.count);
+    }
+  }
 
   // Persistent 1-D grid over kXcds interleaved item lists; see the kernel.
   const int64_t npairs = (int64_t)a->num_seqs * a->num_kv_heads;

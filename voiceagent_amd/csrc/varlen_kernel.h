@@ -12,8 +12,11 @@
 //
 // Tiling (one workgroup = 4 wave64 = 256 lanes): an item is one
 // (sequence, kv head, query block) with all G query heads of the kv group,
-// so its 128 MFMA rows are BQ = 128 / G query positions x G heads.  Each wave
-// owns two 16-row tiles.  Workgroups are persistent: the grid fills the
+// so its 128 MFMA rows are BQ = 128 / G query positions x G heads, row
+// r = position G + head: a short block fills the first rows only.  Wave w
+// owns the 16-row tiles w and w + 4 and leaves out those past the block's
+// last row, so a decoding sequence in a mixed batch (G rows) costs one tile
+// of one wave.  Workgroups are persistent: the grid fills the
 // GPU's workgroup slots once and each workgroup works through a list of
 // items.  Keys stream through LDS in 64-key tiles (K and V row-major,
 // 16-byte chunks XOR-swizzled by row against bank conflicts) over a ring of
@@ -30,6 +33,15 @@
 // With a paged pool, keys j < k_len - q_len are gathered through the block
 // table while the tile is loaded; the new keys come from k/v.  The fused
 // store copies an item's new K/V rows from the staged tiles to slot_mapping.
+//
+// Splitting.  A launch with few items, or with some much longer than the rest
+// (a prompt continuing a long cached prefix, decoding sequences with long
+// contexts beside prompts), would wait for its longest items with most of
+// the chip idle.  Given a workspace, a launch cuts such items' keys into
+// pieces of about (all tiles) / (workgroup slots) tiles (kSplit); a piece
+// writes its rows' unnormalised (m, l, o) in fp32 and varlen_merge_kernel
+// combines them with the log-sum-exp rule.  The plan is made on the device,
+// from the lengths: every workgroup of an XCD computes the same one.
 #pragma once
 
 #include <atomic>
@@ -73,11 +85,39 @@ struct VarlenParams {
   int32_t num_seqs, num_kv_heads;
   FastDiv bs_div, hkv_div;  // block_size, num_kv_heads
   int32_t slot_small;       // num_blocks * block_size <= 2^31: slots divide in 32 bits
+  int32_t block16;          // block_size % 16 == 0: 16 rows from a multiple of 16 share a block
   float k_scale, v_scale;   // FP8 pool: element = code * scale
   int32_t kv_f8;            // the pool holds e4m3 codes (strides in bytes of codes)
+  // Split items (kSplit; all null / 0 without a workspace): per XCD
+  // kSplitSlots pieces, their (m, l) and o, what they belong to, how many.
+  int32_t split;  // host: take the kSplit instantiation
+  float* part_o;
+  float2* part_ml;
+  int4* part_head;
+  int32_t* part_count;
   int32_t has_pro;          // the Qwen3 query prologue runs on every query row
   PrologueParams pro;
 };
+
+// The launch's arguments where they are needed once per item or on uncommon
+// tiles.  Read through a pointer the compiler cannot see through, they are
+// reloaded there (scalar loads) instead of staying in scalar registers
+// through the tile loop, which has none to spare: what is kept beyond them
+// is spilled to vector lanes and read back with v_readlane on every tile.
+// VarlenParams is the kernel's only argument, so it starts the segment.
+typedef const __attribute__((address_space(4))) VarlenParams* ColdArgs;
+__device__ inline ColdArgs cold_args() {
+  ColdArgs a = (ColdArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return a;
+}
+__device__ inline FastDiv cold_div(const __attribute__((address_space(4))) FastDiv& d) {
+  FastDiv r;
+  r.mul = d.mul;
+  r.shift = d.shift;
+  r.d = d.d;
+  return r;
+}
 
 template <bool kBF16>
 struct Mma {
@@ -112,6 +152,30 @@ constexpr int kStages = 2;
 constexpr int kXcds = 8;
 // Lazy-rescale slack of the online softmax, in log2 units (p <= 2^kLazy).
 constexpr float kLazy = 8.0f;
+
+// Splitting: the most pieces of split items on one XCD (the plan needs at
+// most twice the slots it spreads over, and spreads over at most half this
+// number) and the fewest tiles a piece holds (see plan_split in the kernel).
+constexpr int kSplitSlots = 128;
+constexpr int kSplitMinTiles = 2;
+constexpr int kSplitMaxTiles = 1 << 18;  // longer contexts are not split (float division)
+
+// floor(a / b) for 0 <= a < 2^21, b >= 1, through one float product: a + 1/2
+// is at least 1 / (2 b) away from any multiple of b, above the rounding error.
+__device__ inline int small_div(int a, float inv_b) {
+  return (int)(((float)a + 0.5f) * inv_b);
+}
+
+// Inclusive sum over the lanes of a wave (DPP row shifts and broadcasts).
+__device__ inline int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15, rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31, rows 2 and 3
+  return x;
+}
 
 // 16 zero bytes: the DMA source of every lane whose key row is past the end
 // of the visible keys or unmapped, so every tile takes the same number of
@@ -151,8 +215,12 @@ __device__ inline s16x4_t lds_read_tr(const char* base, int off) {
 // kPro: q holds raw projections; each item's query rows are normalised and
 // rotated (Qwen3's q_norm + rotary_emb, prologue.h's arithmetic) in registers
 // at the item's first tile, with positions loaded beside the rows.
-template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce, bool kF8 = false,
-          bool kPro = false>
+//
+// kSplit: the launch has a workspace and may split items (an instantiation of
+// its own: the plan's state costs the others scalar registers, 1 us of 41 on
+// a launch of 32 prompts).
+template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce, bool kF8, bool kPro,
+          bool kSplit>
 __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(VarlenParams p) {
   constexpr int BQ = kRowsPerWG / G;       // query positions per workgroup
   constexpr int DS = D / 32;               // k-steps of the S^T MFMA
@@ -187,7 +255,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   using ET = std::conditional_t<kBF16, BF16, F16>;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: addresses stay scalar
   const int lane = tid & 63;
   const int r16 = lane & 15;
   const int g4 = lane >> 4;
@@ -258,15 +326,96 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   }
 
   struct Item {
-    int h, qb, q0, ql, k0, kl;
-    int pos0, pos_end, diag, pool_prefix, kend, ntiles;
-    int64_t new_base, table_row;
+    int s, h, qb;        // sequence, kv head, query block
+    int q0, ql, k0, kl;  // the sequence's first query and key, its lengths
+    int t0, t1;          // its key tiles, or the piece's
+    int slot, npc;       // piece of a split item: its partial's slot (-1: whole), pieces if first
   };
+  // What follows from an item: the keys that come from the pool, and the end
+  // of the keys its rows see (bottom-right aligned when causal).
+  const bool has_k = !kPaged || p.k != nullptr;
+  auto prefix_of = [&](const Item& it) { return kPaged ? (has_k ? it.kl - it.ql : it.kl) : 0; };
+  auto kend_of = [&](const Item& it) {
+    return kCausal ? max(0, min(it.kl, it.kl - it.ql + min(it.ql, it.qb * BQ + BQ))) : it.kl;
+  };
+  // ---- splitting (kSplit) ----
+  // The items' tiles on this XCD over its slots (fewer where there are many
+  // items, each of which costs a slot its set-up and epilogue) give the tiles
+  // of a piece; an item longer than that by a quarter is cut into equal
+  // pieces of at most that many plus a quarter.  tile_sum is an upper bound
+  // of the tiles (prefix tiles rounded up to quarters, one per item for the
+  // rest), so split items have at most 2 tile_sum / piece <= kSplitSlots
+  // pieces.
+  // (Stores of the plan's words are uniform, by all lanes of a wave: a branch
+  // on the lane in this walk would make every value after it divergent, the
+  // DMAs' scalar bases among them.)
+  int piece = 0;  // tiles of a piece; 0: nothing is split
+  float piece_inv = 0.f;
+  auto tiles_at = [&](int ql, int kl, int lv) {
+    const int kend = kCausal ? max(0, min(kl, kl - ql + min(ql, lv * BQ + BQ))) : kl;
+    return (kend + kKeyTile - 1) / kKeyTile;
+  };
+  auto plan_split = [&]() {
+    const int nt = lnq > 0 ? (lkl + kKeyTile - 1) / kKeyTile : 0;
+    const int prefix = max(lkl - lql, 0);
+    int sum = 0;
+    if (lnq > 0)
+      sum = kCausal ? lnq * ((prefix + 15) / 16) / 4 + lnq * (lnq + 1) / 2 * BQ / kKeyTile + lnq + 1
+                    : lnq * nt;
+    if (__builtin_amdgcn_ballot_w64(nt >= kSplitMaxTiles || lnq > 1024 || sum >= (1 << 24)) != 0) return;
+    const int tile_sum = __builtin_amdgcn_readlane(wave_scan(sum), 63);
+    const int items = __builtin_amdgcn_readlane(wave_scan(lnq), 63);
+    const int over = min(max(nslots - items / 4, (nslots + 1) / 2), kSplitSlots / 2);
+    const int pc = max(__builtin_amdgcn_readfirstlane((tile_sum + over - 1) / over), kSplitMinTiles);
+    if (__builtin_amdgcn_ballot_w64(nt > pc + pc / 4) != 0) {
+      piece = pc;
+      piece_inv = 1.f / (float)pc;
+    }
+  };
+  if constexpr (kSplit) {
+    if (lane_pairs) plan_split();
+    if (piece == 0 && wslot == 0 && wave == 0) p.part_count[xcd] = 0;
+  }
   int round = 0;                         // this workgroup's next round
   int lev = nqb - 1, cum = 0;            // lane_pairs walk: level and items above it
+  int slots = 0;                         // pieces of split items above it
   auto next_item = [&](Item& it) -> bool {
     int ksel, qb;
-    if (lane_pairs) {
+    it.slot = -1;
+    it.npc = 1;
+    int pj = 0, pn = 1;  // this piece of its item, pieces of the item
+    if (kSplit && piece > 0) {
+      const int li = (int)item_index(round);
+      int pc = 0, inc = 0;
+      while (lev >= 0) {
+        // Pieces of every pair's item at this level, and their running sums:
+        // all pieces in the low half, those of split items in the high half.
+        pc = lnq > lev
+                 ? max(1, small_div(tiles_at(lql, lkl, lev) + piece - 1 - piece / 4, piece_inv))
+                 : 0;
+        inc = wave_scan(pc + (pc > 1 ? pc << 16 : 0));
+        const int all = __builtin_amdgcn_readlane(inc, 63);
+        if (li < cum + (all & 0xffff)) break;
+        cum += all & 0xffff;
+        slots += (int)((uint32_t)all >> 16);
+        --lev;
+      }
+      if (lev < 0) {
+        if (wslot == 0 && wave == 0) p.part_count[xcd] = slots;
+        return false;
+      }
+      ++round;
+      const int rem = li - cum;
+      const int end = inc & 0xffff;
+      ksel = __builtin_ctzll(__builtin_amdgcn_ballot_w64(rem < end && rem >= end - pc));
+      pn = __builtin_amdgcn_readlane(pc, ksel);
+      pj = rem - (__builtin_amdgcn_readlane(end, ksel) - pn);
+      if (pn > 1) {
+        it.slot = slots + (int)((uint32_t)__builtin_amdgcn_readlane(inc, ksel) >> 16) - pn + pj;
+        it.npc = pj == 0 ? pn : 0;
+      }
+      qb = lev;
+    } else if (lane_pairs) {
       const int64_t li = item_index(round);
       // Levels are walked downwards once over the workgroup's life: the
       // list indices of its rounds increase.
@@ -285,8 +434,6 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0));
       ksel = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lnq > lev && below == rem));
       qb = lev;
-      const int pair = xcd + kXcds * ksel;
-      it.h = (int)fast_mod((uint32_t)pair, p.hkv_div);
     } else {
       for (;;) {
         if (item_index(round) >= total) return false;
@@ -296,24 +443,24 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
         qb = __builtin_amdgcn_readlane(lnq, ksel);
         if (qb * BQ < __builtin_amdgcn_readlane(lql, ksel)) break;  // else past the end
       }
-      it.h = (int)fast_mod((uint32_t)__builtin_amdgcn_readlane(lpair, ksel), p.hkv_div);
     }
     const int pair = lane_pairs ? xcd + kXcds * ksel : __builtin_amdgcn_readlane(lpair, ksel);
-    const int s = (int)fast_div((uint32_t)pair, p.hkv_div);
+    it.s = (int)fast_div((uint32_t)pair, p.hkv_div);
+    it.h = pair - it.s * p.num_kv_heads;
     it.qb = qb;
     it.q0 = __builtin_amdgcn_readlane(lq0, ksel);
     it.ql = __builtin_amdgcn_readlane(lql, ksel);
     it.k0 = __builtin_amdgcn_readlane(lk0, ksel);
     it.kl = __builtin_amdgcn_readlane(lkl, ksel);
-    it.pos0 = qb * BQ;
-    it.pos_end = min(it.ql, it.pos0 + BQ);
-    it.diag = it.kl - it.ql;  // bottom-right alignment offset
-    it.pool_prefix = kPaged ? (p.k != nullptr ? it.kl - it.ql : it.kl) : 0;
-    it.kend = kCausal ? max(0, min(it.kl, it.diag + it.pos_end)) : it.kl;
-    it.ntiles = (it.kend + kKeyTile - 1) / kKeyTile;
-    // Keys from k/v: key j is row new_base + j of k and v.
-    it.new_base = kPaged ? (int64_t)it.q0 - it.pool_prefix : (int64_t)it.k0;
-    it.table_row = (int64_t)s * p.t_sb;
+    const int nt = tiles_at(it.ql, it.kl, qb);
+    it.t0 = 0;
+    it.t1 = nt;
+    if (kSplit && pn > 1) {
+      const int q = __builtin_amdgcn_readfirstlane(small_div(nt, 1.f / (float)pn));
+      const int r = nt - q * pn;
+      it.t0 = pj * q + min(pj, r);
+      it.t1 = it.t0 + q + (pj < r ? 1 : 0);
+    }
     return true;
   };
 
@@ -322,125 +469,182 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   const uint32_t code_base = __builtin_amdgcn_readfirstlane(
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)s_code);
 
-  // ---- DMA of key tile [kb, kb + 64) into stage st ----
-  // (h, pool_prefix, kend, new_base, table_row) are the item's; all uniform.
-  // Wave w fills 1 KiB blocks w NI .. w NI + NI - 1 of the K and V tiles;
-  // lane l of a block writes row RPI * block + l / CPR, chunk position l % CPR,
-  // so it reads logical chunk (l % CPR) ^ swz(row) of that key.  Every lane
-  // issues exactly 2 NI DMAs per tile.
-  uint32_t koff[NI], voff[NI];  // per-lane byte offsets inside a tile of k/v rows
+  // ---- DMA of a key tile [kb, kb + 64) into a stage ----
+  // Wave w fills 1 KiB blocks w NI .. w NI + NI - 1 of the K and V tiles,
+  // which hold the tile's rows 16 w .. 16 w + 15; lane l of block i writes
+  // row RPI i + l / CPR of them, chunk position l % CPR, so it reads logical
+  // chunk (l % CPR) ^ swz(row) of that key.
+  static_assert(NI * RPI == 16, "a wave stages 16 rows of a tile");
+  uint32_t koff[NI], voff[NI];  // per-lane byte offsets inside the wave's 16 k/v rows
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int row = (wave * NI + i) * RPI + lane / CPR;
+    const int row = RPI * i + lane / CPR;
     const int chunk = (lane % CPR) ^ swz<D>(row);
     koff[i] = (uint32_t)(row * p.k_st + chunk * 16);
     voff[i] = (uint32_t)(row * p.v_st + chunk * 16);
   }
+  // The same inside 16 pool rows of one block (K and V alike): swz is linear
+  // over XOR, so the lane's chunk of row RPI i + r is c0 ^ swz(RPI i).
+  const uint32_t pool_row = kPaged ? (uint32_t)(lane / CPR) * (uint32_t)p.s_slot : 0u;
+  const uint32_t pool_c0 = (uint32_t)(((lane % CPR) ^ swz<D>(lane / CPR)) << 4);
+  auto pool_off = [&](int i) {
+    return (pool_c0 ^ (uint32_t)(swz<D>(RPI * i) << 4)) + pool_row +
+           (uint32_t)(i * RPI) * (uint32_t)p.s_slot;
+  };
+  // FP8 pool: a wave's 16 code rows (unswizzled, CRPI rows an instruction).
+  const uint32_t code_lane =
+      kF8 ? (uint32_t)(lane / CCPR) * (uint32_t)p.s_slot + (uint32_t)(lane % CCPR) * 16u : 0u;
+  const uint32_t code_dst = code_base + (uint32_t)(wave * NIC * 1024);
+
+  // The cursor of the tiles being requested, one step ahead of the tiles
+  // being reduced: it runs through the current item's tiles and on into the
+  // next item's.  A whole tile of k/v rows, or (block16: a wave's 16 rows lie
+  // in one block) of pool rows, is an easy one: instruction i copies RPI rows
+  // from a uniform base plus lane offsets, with no load or per-lane address
+  // of its own, so it can be issued between the MFMAs.  Every other tile
+  // takes issue_hard.
+  struct Cursor {
+    int t, end;           // next tile to request, the item's last + 1
+    int prefix, kend;
+    int h, s;
+    int64_t base;         // key j of k/v is row base + j
+    int row0;             // `rows` holds the pool rows of tiles [row0, row0 + 64)
+  };
+  Cursor cu;
+  int64_t rows = -1;
+  uint2 pend = make_uint2(0u, 0u);  // raw block ids that `rows` takes next
+  auto cursor_to = [&](const Item& it) {
+    cu.t = it.t0;
+    cu.prefix = prefix_of(it);
+    cu.kend = kend_of(it);
+    cu.end = it.t1;
+    cu.h = it.h;
+    cu.s = it.s;
+    cu.base = kPaged ? (int64_t)it.q0 - cu.prefix : (int64_t)it.k0;
+    cu.row0 = it.t0;
+  };
+  // ---- pool rows (block16) ----
+  // Lane l of `rows` holds the pool byte offset of the wave's 16 rows of tile
+  // row0 + l (-1: a block id outside the pool).  Block ids are requested 64
+  // tiles at a time and a tile ahead of their use, so no tile waits for them
+  // (looked up as the tile was requested, each pool tile cost a second
+  // dependent round trip: 4 prompts of 200-300 tokens over prefixes of 2K-8K
+  // took 357 us, 2.8 us a tile, and 260 with the ids ahead); they stay raw
+  // words until a later step's tile wait has passed.  Columns past the table
+  // read block 0.
+  auto load_ids = [&](int s, int t0, int prefix) {
+    const ColdArgs ca = cold_args();
+    pend = make_uint2(0u, 0u);
+    const int tok = (t0 + lane) * kKeyTile + 16 * wave;
+    const int col = (int)fast_div((uint32_t)tok, cold_div(ca->bs_div));
+    if (tok < prefix && col < ca->table_width) {
+      const uint32_t* const w = reinterpret_cast<const uint32_t*>(ca->table);
+      const int i64 = ca->table_i64;
+      const int64_t e = ((int64_t)s * ca->t_sb + col) << i64;
+      pend.x = w[e];
+      pend.y = w[e + i64];
+    }
+  };
+  auto take_ids = [&](int t0) {  // the requested ids are those of the cursor's tiles from t0 on
+    cu.row0 = t0;
+    if (cu.prefix <= t0 * kKeyTile) return;  // no pool rows there
+    const ColdArgs ca = cold_args();
+    const int64_t bid = ca->table_i64 ? (int64_t)(((uint64_t)pend.y << 32) | pend.x)
+                                      : (int64_t)(int32_t)pend.x;
+    const uint32_t tok = (uint32_t)((t0 + lane) * kKeyTile + 16 * wave);
+    rows = -1;
+    if (bid >= 0 && bid < ca->num_blocks)
+      rows = bid * ca->s_blk + (int64_t)fast_mod(tok, cold_div(ca->bs_div)) * ca->s_slot +
+             cu.h * ca->s_head;
+  };
+  // What `rows` will need next: the item's following 64 tiles, or the next
+  // item's first.
+  auto request_ids = [&](bool has_next, const Item& nxt) {
+    if constexpr (!kPaged) return;
+    if (cu.end - cu.row0 > 64) {
+      if (cu.prefix > (cu.row0 + 64) * kKeyTile) load_ids(cu.s, cu.row0 + 64, cu.prefix);
+    } else if (has_next && prefix_of(nxt) > 0) {
+      load_ids(nxt.s, nxt.t0, prefix_of(nxt));
+    }
+  };
+
+  // How the cursor's tile is requested.
+  enum { kNone, kRows, kPool, kCodes };
+  struct Easy {
+    int kind;
+    const char* kb;  // the wave's first row
+    const char* vb;
+  };
   const char* zero_row = reinterpret_cast<const char*>(&kZeroRow);
-  auto issue_tile = [&](int h, int pool_prefix, int kend, int64_t new_base, int64_t table_row,
-                        int kb, int st) {
+  auto issue_hard = [&](int64_t row, int st) {
+    const ColdArgs ca = cold_args();
     const uint32_t dst0 = lds_base + (uint32_t)(st * 2 * TILE_B + wave * NI * 1024);
-    if (kb >= pool_prefix && kb + kKeyTile <= kend) {
-      // Whole tile from k/v: uniform bases, constant lane offsets.
-      const char* kbase = uniform_ptr(p.k + (new_base + kb) * p.k_st + h * p.k_sh);
-      const char* vbase = uniform_ptr(p.v + (new_base + kb) * p.v_st + h * p.v_sh);
-      if constexpr (kv_once) {
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          dma16_nt(koff[i], kbase, dst0 + i * 1024);
-          dma16_nt(voff[i], vbase, dst0 + TILE_B + i * 1024);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          dma16(koff[i], kbase, dst0 + i * 1024);
-          dma16(voff[i], vbase, dst0 + TILE_B + i * 1024);
-        }
-      }
-      return;
-    }
-    // Tile with pool keys or past kend: per-lane addresses; rows past kend
-    // or with an unmapped block read kZeroRow.  The lane's first row is
-    // made opaque so that the per-lane address arithmetic stays here
-    // instead of being hoisted out of the tile loop into live registers.
-    // Block ids are loaded as raw words and widened after the last load, and
-    // every address is formed before the first DMA: a register still
-    // awaiting its load when a DMA has been issued would make the compiler's
-    // wait for it also wait for that DMA.
-    int row0 = wave * NI * RPI + lane / CPR;
+    const int kb = cu.t * kKeyTile;
+    const FastDiv bs_div = cold_div(ca->bs_div);
+    // Per-lane addresses; rows past kend or with an unmapped block read
+    // kZeroRow.  The lane's first row is made opaque so that the address
+    // arithmetic stays here instead of being hoisted out of the tile loop
+    // into live registers.  Block ids (other block sizes; with block16 the
+    // wave's 16 rows start at pool offset `row`) are loaded as raw words and widened after the last
+    // load, and every address is formed before the first DMA: a register
+    // still awaiting its load when a DMA has been issued would make the
+    // compiler's wait for it also wait for that DMA.
+    int row0 = 16 * wave + lane / CPR;
     asm volatile("" : "+v"(row0));
-    uint2 braw[NI];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) braw[i] = make_uint2(0u, 0u);
-    if (kPaged && !kF8 && kb < pool_prefix) {
-      int64_t e[NI];
-      bool ok[NI];
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int j = kb + row0 + i * RPI;
-        const int col = (int)fast_div((uint32_t)j, p.bs_div);
-        ok[i] = j < pool_prefix && j < kend && col < p.table_width;
-        e[i] = table_row + col;
-      }
-      if (p.table_i64) {
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-          if (ok[i]) braw[i] = reinterpret_cast<const uint2*>(p.table)[e[i]];
+    // Address of the 16 bytes at byte column `c16` of token j's pool row.
+    auto pool_at = [&](int j, const uint2& raw, int c16, const char*& ka, const char*& va_) {
+      int64_t off = row;
+      if (ca->block16) {
+        if (off >= 0) off += (j & 15) * ca->s_slot + c16;
       } else {
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-          if (ok[i]) braw[i].x = reinterpret_cast<const uint32_t*>(p.table)[e[i]];
+        const int64_t bid = ca->table_i64 ? (int64_t)(((uint64_t)raw.y << 32) | raw.x)
+                                          : (int64_t)(int32_t)raw.x;
+        off = -1;
+        if (bid >= 0 && bid < ca->num_blocks)
+          off = bid * ca->s_blk + (int64_t)fast_mod((uint32_t)j, bs_div) * ca->s_slot +
+                cu.h * ca->s_head + c16;
       }
-    }
-    // FP8 pool: the tile's pool rows as codes.  Lane l of code instruction i
-    // copies chunk l % CCPR of code row (wave NIC + i) CRPI + l / CCPR.
+      if (off >= 0) {
+        ka = ca->kp + off;
+        va_ = ca->vp + off;
+      }
+    };
+    auto raw_id = [&](int j, uint2& raw) {
+      raw = make_uint2(0u, 0u);
+      if (!ca->block16) {
+        const int col = (int)fast_div((uint32_t)j, bs_div);
+        if (j < cu.prefix && j < cu.kend && col < ca->table_width) {
+          const int i64 = ca->table_i64;
+          const int64_t e = ((int64_t)cu.s * ca->t_sb + col) << i64;
+          const uint32_t* const w = reinterpret_cast<const uint32_t*>(ca->table);
+          raw.x = w[e];
+          raw.y = w[e + i64];
+        }
+      }
+    };
     const char* kc[kF8 ? NIC : 1];
     const char* vc[kF8 ? NIC : 1];
     if constexpr (kF8) {
+      // The tile's pool rows as codes: lane l of code instruction i copies
+      // chunk l % CCPR of code row (wave NIC + i) CRPI + l / CCPR.
+      int crow0 = 16 * wave + lane / CCPR;
+      asm volatile("" : "+v"(crow0));
+      uint2 craw[NIC];
+#pragma unroll
+      for (int i = 0; i < NIC; ++i) raw_id(kb + crow0 + i * CRPI, craw[i]);
 #pragma unroll
       for (int i = 0; i < NIC; ++i) {
+        const int j = kb + crow0 + i * CRPI;
         kc[i] = zero_row;
         vc[i] = zero_row;
+        if (j < cu.prefix && j < cu.kend) pool_at(j, craw[i], (lane % CCPR) * 16, kc[i], vc[i]);
       }
-      if (kb < pool_prefix) {
-        int crow0 = wave * NIC * CRPI + lane / CCPR;
-        asm volatile("" : "+v"(crow0));
-        uint2 craw[NIC];
-        bool cok[NIC];
-        int64_t ce[NIC];
+    }
+    uint2 braw[NI];
 #pragma unroll
-        for (int i = 0; i < NIC; ++i) {
-          const int j = kb + crow0 + i * CRPI;
-          const int col = (int)fast_div((uint32_t)j, p.bs_div);
-          cok[i] = j < pool_prefix && j < kend && col < p.table_width;
-          ce[i] = table_row + col;
-          craw[i] = make_uint2(0u, 0u);
-        }
-        if (p.table_i64) {
-#pragma unroll
-          for (int i = 0; i < NIC; ++i)
-            if (cok[i]) craw[i] = reinterpret_cast<const uint2*>(p.table)[ce[i]];
-        } else {
-#pragma unroll
-          for (int i = 0; i < NIC; ++i)
-            if (cok[i]) craw[i].x = reinterpret_cast<const uint32_t*>(p.table)[ce[i]];
-        }
-        // As for 16-bit rows: a column at or past the table width keeps
-        // block id 0 (read as block 0, the TTS padding semantics).
-#pragma unroll
-        for (int i = 0; i < NIC; ++i) {
-          const int j = kb + crow0 + i * CRPI;
-          const int64_t bid = p.table_i64 ? (int64_t)(((uint64_t)craw[i].y << 32) | craw[i].x)
-                                          : (int64_t)(int32_t)craw[i].x;
-          if (j < pool_prefix && j < kend && bid >= 0 && bid < p.num_blocks) {
-            const int64_t off = bid * p.s_blk +
-                                (int64_t)fast_mod((uint32_t)j, p.bs_div) * p.s_slot +
-                                h * p.s_head + (lane % CCPR) * 16;
-            kc[i] = p.kp + off;
-            vc[i] = p.vp + off;
-          }
-        }
-      }
+    for (int i = 0; i < NI; ++i) {
+      braw[i] = make_uint2(0u, 0u);
+      if (kPaged && !kF8) raw_id(kb + row0 + i * RPI, braw[i]);
     }
     const char* ka[NI];
     const char* va_[NI];
@@ -451,52 +655,100 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       const int j = kb + row;
       ka[i] = zero_row;
       va_[i] = zero_row;
-      if (j < kend) {
-        if (kPaged && j < pool_prefix) {
+      if (j < cu.kend) {
+        if (kPaged && j < cu.prefix) {
           // An FP8 pool row is staged by the code copy and its conversion.
-          if constexpr (kF8) continue;
-          const int64_t bid = p.table_i64 ? (int64_t)(((uint64_t)braw[i].y << 32) | braw[i].x)
-                                          : (int64_t)(int32_t)braw[i].x;
-          if (bid >= 0 && bid < p.num_blocks) {
-            const int64_t off = bid * p.s_blk + (int64_t)fast_mod((uint32_t)j, p.bs_div) * p.s_slot +
-                                h * p.s_head + chunk * 16;
-            ka[i] = p.kp + off;
-            va_[i] = p.vp + off;
-          }
+          if constexpr (!kF8) pool_at(j, braw[i], chunk * 16, ka[i], va_[i]);
         } else {
-          ka[i] = p.k + (new_base + j) * p.k_st + h * p.k_sh + chunk * 16;
-          va_[i] = p.v + (new_base + j) * p.v_st + h * p.v_sh + chunk * 16;
+          ka[i] = ca->k + (cu.base + j) * ca->k_st + cu.h * ca->k_sh + chunk * 16;
+          va_[i] = ca->v + (cu.base + j) * ca->v_st + cu.h * ca->v_sh + chunk * 16;
         }
       }
     }
-    if constexpr (kv_once) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
+    for (int i = 0; i < NI; ++i) {
+      if constexpr (kv_once) {
         dma16_nt(ka[i], dst0 + i * 1024);
         dma16_nt(va_[i], dst0 + TILE_B + i * 1024);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
+      } else {
         dma16(ka[i], dst0 + i * 1024);
         dma16(va_[i], dst0 + TILE_B + i * 1024);
       }
     }
     if constexpr (kF8) {
-      if (kb < pool_prefix) {
-        const uint32_t cdst = code_base + (uint32_t)(wave * NIC * 1024);
+      if (kb < cu.prefix) {
 #pragma unroll
         for (int i = 0; i < NIC; ++i) {
-          dma16(kc[i], cdst + i * 1024);
-          dma16(vc[i], cdst + CODE_B + i * 1024);
+          dma16(kc[i], code_dst + i * 1024);
+          dma16(vc[i], code_dst + CODE_B + i * 1024);
         }
+      }
+    }
+  };
+  // Requests the cursor's tile into stage st, or, when it is an easy one,
+  // says how (easy_issue then does, one instruction pair at a time).
+  auto issue = [&](int st) -> Easy {
+    Easy e;
+    e.kind = kNone;
+    e.kb = e.vb = nullptr;
+    const int kb = cu.t * kKeyTile;
+    if (kb >= cu.prefix && kb + kKeyTile <= cu.kend) {
+      const int64_t row = cu.base + kb + 16 * wave;
+      e.kind = kRows;
+      e.kb = uniform_ptr(p.k + row * p.k_st + cu.h * p.k_sh);
+      e.vb = uniform_ptr(p.v + row * p.v_st + cu.h * p.v_sh);
+      return e;
+    }
+    int64_t row = -1;
+    if (kPaged && kb < cu.prefix) {
+      const int l = cu.t - cu.row0;
+      row = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(rows >> 32), l) << 32) |
+                      (uint32_t)__builtin_amdgcn_readlane((int)rows, l));
+      if (kb + kKeyTile <= min(cu.prefix, cu.kend) && row >= 0 && p.block16) {
+        e.kind = kF8 ? kCodes : kPool;
+        e.kb = uniform_ptr(p.kp + row);
+        e.vb = uniform_ptr(p.vp + row);
+        return e;
+      }
+    }
+    issue_hard(row, st);
+    return e;
+  };
+  auto easy_issue = [&](const Easy& e, int i, uint32_t dst) {  // 16-bit rows
+    if constexpr (kv_once) {
+      dma16_nt(koff[i], e.kb, dst + i * 1024);
+      dma16_nt(voff[i], e.vb, dst + TILE_B + i * 1024);
+    } else if (!kPaged || kF8 || e.kind == kRows) {
+      dma16(koff[i], e.kb, dst + i * 1024);
+      dma16(voff[i], e.vb, dst + TILE_B + i * 1024);
+    } else {
+      const uint32_t o = pool_off(i);
+      dma16(o, e.kb, dst + i * 1024);
+      dma16(o, e.vb, dst + TILE_B + i * 1024);
+    }
+  };
+  auto easy_codes = [&](const Easy& e, int i) {
+    const int64_t step = (int64_t)(i * CRPI) * p.s_slot;
+    dma16(code_lane, e.kb + step, code_dst + i * 1024);
+    dma16(code_lane, e.vb + step, code_dst + CODE_B + i * 1024);
+  };
+  auto issue_now = [&](const Easy& e, int st) {  // all of an easy tile at once
+    const uint32_t dst = lds_base + (uint32_t)(st * 2 * TILE_B + wave * NI * 1024);
+    if (e.kind == kRows || e.kind == kPool) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) easy_issue(e, i, dst);
+    }
+    if constexpr (kF8) {
+      if (e.kind == kCodes) {
+#pragma unroll
+        for (int i = 0; i < NIC; ++i) easy_codes(e, i);
       }
     }
   };
 
   // ---- query rows and store slots of an item ----
-  // Two 16-row tiles per wave: row 16 (2 wave + tt) + r16 of the block is
-  // query position pos0 + row % BQ of head h G + row / BQ.
+  // Two 16-row tiles per wave: row 16 (wave + 4 tt) + r16 of the block is
+  // query position pos0 + row / G of head h G + row % G.
   uint4 qreg[2][DS];
   // kPro: the rotary position of each of the lane's two query rows (the row
   // of the item's last query for rows past the end, whose output is unused).
@@ -504,19 +756,19 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   auto load_q = [&](const Item& it) {
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
-      const int row = 16 * (2 * wave + tt) + r16;
-      const int qpos = it.pos0 + row % BQ;
-      const int qhead = it.h * G + row / BQ;
+      const int row = 16 * (wave + 4 * tt) + r16;
+      const int qpos = it.qb * BQ + row / G;
+      const int qhead = it.h * G + row % G;
       if constexpr (kPro)
         qrot[tt] = load_index(p.pro.pos, (int64_t)it.q0 + (qpos < it.ql ? qpos : it.ql - 1),
                               p.pro.pos_i64);
+      const char* const src = p.q + (int64_t)(it.q0 + qpos) * p.q_st +
+                              (int64_t)qhead * p.q_sh + g4 * 16;
 #pragma unroll
-      for (int ds = 0; ds < DS; ++ds) {
-        if (qpos < it.ql)
-          qreg[tt][ds] = ld16(p.q + (int64_t)(it.q0 + qpos) * p.q_st +
-                              (int64_t)qhead * p.q_sh + (32 * ds + 8 * g4) * 2);
-        else
-          qreg[tt][ds] = make_uint4(0, 0, 0, 0);
+      for (int ds = 0; ds < DS; ++ds) qreg[tt][ds] = make_uint4(0, 0, 0, 0);
+      if (qpos < it.ql) {
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) qreg[tt][ds] = ld16(src + 64 * ds);
       }
     }
   };
@@ -535,7 +787,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   constexpr int RPS = 64 / CPR;  // rows per store step
   constexpr int NSTEP = (BQ * CPR + kVarlenThreads - 1) / kVarlenThreads;
   static_assert(NSTEP * RPS <= 64, "one slot lane per row");
-  const bool fused_store = kPaged && p.slots != nullptr;
+  const bool fused_store = kPaged && !kF8 && p.slots != nullptr;  // FP8: a launch of its own
   auto st_base = [&](int k) {  // first block row of store step k (BQ: none)
     const int e0 = k * kVarlenThreads + 64 * wave;
     return e0 < BQ * CPR ? e0 / CPR : BQ;
@@ -543,8 +795,8 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   const int st_row = lane < NSTEP * RPS ? min(st_base(lane / RPS) + lane % RPS, BQ) : BQ;
   auto load_slot = [&](const Item& it) -> uint2 {
     uint2 raw = make_uint2(~0u, ~0u);
-    if (fused_store && it.pos0 + st_row < it.pos_end) {
-      const int64_t i = (int64_t)it.q0 + it.pos0 + st_row;
+    if (fused_store && it.qb * BQ + st_row < min(it.ql, it.qb * BQ + BQ)) {
+      const int64_t i = (int64_t)it.q0 + it.qb * BQ + st_row;
       if (p.slot_i64)
         raw = reinterpret_cast<const uint2*>(p.slots)[i];
       else
@@ -559,29 +811,40 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
 
   Item cur, nxt;
   if (!next_item(cur)) return;
-  if (cur.ntiles > 0)
-    issue_tile(cur.h, cur.pool_prefix, cur.kend, cur.new_base, cur.table_row, 0, 0);
+  cursor_to(cur);
+  if (kPaged && cu.prefix > 0) {
+    load_ids(cur.s, cur.t0, cu.prefix);
+    take_ids(cur.t0);
+  }
+  if (cu.t < cu.end) {
+    issue_now(issue(0), 0);
+    ++cu.t;
+  }
   load_q(cur);
   uint2 st_slot = load_slot(cur);
   int stage = 0;  // stage holding the current item's next tile to reduce
 
   for (;;) {
     const bool has_next = next_item(nxt);
+    request_ids(has_next, nxt);
 
-    int qpos[2], qhead[2], lim[2];
+    const int pos0 = cur.qb * BQ;
+    const int nrows = (min(cur.ql, pos0 + BQ) - pos0) * G;  // MFMA rows of the block in use
+    const int prefix = prefix_of(cur);
+    const int kend = kend_of(cur);
+    const int tend = cur.t1;
+    int lim[2];
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
-      const int row = 16 * (2 * wave + tt) + r16;
-      qhead[tt] = cur.h * G + row / BQ;
-      qpos[tt] = cur.pos0 + row % BQ;
       // Visible keys per row: j < lim[tt].  Rows past the end of the
       // sequence have zero queries; their outputs are never written.
-      lim[tt] = kCausal ? min(cur.kend, cur.diag + qpos[tt] + 1) : cur.kend;
+      const int qpos = pos0 + (16 * (wave + 4 * tt) + r16) / G;
+      lim[tt] = kCausal ? min(kend, cur.kl - cur.ql + qpos + 1) : kend;
     }
-    // Tiles ending at or below lim_lo (the smallest limit in the block) need
-    // no mask.
-    const int lim_lo = kCausal ? min(cur.kend, cur.diag + cur.pos0 + 1) : cur.kend;
-    const int st_key0 = cur.pool_prefix + cur.pos0;  // key of the block's first row
+    // Tiles ending at or below lim_lo (the smallest limit of the wave's rows)
+    // need no mask.
+    const int lim_lo = kCausal ? min(kend, cur.kl - cur.ql + pos0 + 16 * wave / G + 1) : kend;
+    const int st_key0 = prefix + pos0;  // key of the block's first row
 
     float m[2] = {-1.0e30f, -1.0e30f};
     float l[2] = {0.f, 0.f};
@@ -595,7 +858,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
         for (int dt = 0; dt < DT; ++dt) o[tt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
 
-    for (int t = 0; t < cur.ntiles; ++t) {
+    for (int t = cur.t0; t < tend; ++t) {
       const int kb = t * kKeyTile;
       // Tile t (and, in order, everything issued before it) has landed once
       // nothing is pending; the barrier makes every wave's part of it
@@ -604,9 +867,9 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       // item's first tile.
       wait_vmcnt<0>();
       __syncthreads();
-      // The query rows and slot were loaded before the wait: make the
-      // compiler's own wait for them fall here, before the next DMA, where
-      // it is free (a later wait would also stall on that DMA).
+      // The query rows, the slot and block ids were loaded before the wait:
+      // make the compiler's own wait for them fall here, before the next
+      // DMA, where it is free (a later wait would also stall on that DMA).
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
@@ -614,6 +877,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
           asm volatile("" ::"v"(qreg[tt][ds].x), "v"(qreg[tt][ds].y), "v"(qreg[tt][ds].z),
                        "v"(qreg[tt][ds].w));
       asm volatile("" ::"v"(st_slot.x), "v"(st_slot.y));
+      if constexpr (kPaged) asm volatile("" ::"v"(pend.x), "v"(pend.y));
       // Qwen3 query prologue on the item's rows, in the B-operand layout:
       // lane (r16, g4) holds elements 32 ds + 8 g4 + e of its row (ds < DS,
       // e < 8), so element i < D/2 and its rotary partner i + D/2 sit in the
@@ -625,7 +889,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       // the output accumulators take after this block; the weights come
       // from LDS.
       if constexpr (kPro) {
-        if (t == 0) {
+        if (t == cur.t0) {
           static_assert(DS % 2 == 0, "rotary halves");
           constexpr int HD = DS / 2;
           f32x4_t cv[2][HD][2], sv[2][HD][2];
@@ -714,13 +978,13 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       // stage (16-byte chunks at their swizzled positions), then free the
       // code area for the next tile's copy below.
       if constexpr (kF8) {
-        if (kb < cur.pool_prefix) {
+        if (kb < prefix) {
           char* const s_kt = s_kv + stage * 2 * TILE_B;
           for (int e = tid; e < 2 * kKeyTile * CCPR; e += kVarlenThreads) {
             const int is_v = e >= kKeyTile * CCPR ? 1 : 0;
             const int rc = e - is_v * kKeyTile * CCPR;
             const int r = rc / CCPR, c = rc % CCPR;
-            if (kb + r < cur.pool_prefix) {
+            if (kb + r < prefix) {
               const uint4 codes = lds_read16(s_code + is_v * CODE_B, r * D + c * 16);
               const float sc = is_v ? p.v_scale : p.k_scale;
               char* const dst = s_kt + is_v * TILE_B + r * ROWB;
@@ -740,26 +1004,27 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
         }
       }
       // The next tile (this item's tile t + 1, or the next item's first)
-      // goes to the other stage.  A whole tile from k/v is issued in NI
-      // pairs spread over the S^T loop below: issued back to back, its DMAs
-      // stall the wave on the vector memory queue for as long as the
-      // MFMAs of half a tile take.  Other tiles are issued here.
-      const bool same = t + 1 < cur.ntiles;
-      const bool next_tile = same || (has_next && nxt.ntiles > 0);
-      const int n_h = same ? cur.h : nxt.h;
-      const int n_prefix = same ? cur.pool_prefix : nxt.pool_prefix;
-      const int n_kend = same ? cur.kend : nxt.kend;
-      const int64_t n_base = same ? cur.new_base : nxt.new_base;
-      const int n_kb = same ? kb + kKeyTile : 0;
-      const bool spread = next_tile && n_kb >= n_prefix && n_kb + kKeyTile <= n_kend;
-      const char* n_kbase = nullptr;
-      const char* n_vbase = nullptr;
-      if (spread) {
-        n_kbase = uniform_ptr(p.k + (n_base + n_kb) * p.k_st + n_h * p.k_sh);
-        n_vbase = uniform_ptr(p.v + (n_base + n_kb) * p.v_st + n_h * p.v_sh);
-      } else if (next_tile) {
-        issue_tile(n_h, n_prefix, n_kend, n_base, same ? cur.table_row : nxt.table_row, n_kb,
-                   stage ^ 1);
+      // goes to the other stage.  An easy tile is issued in pairs of DMAs
+      // spread over the S^T loop below: issued back to back, they stall the
+      // wave on the vector memory queue for as long as the MFMAs of half a
+      // tile take.  Other tiles are issued here.
+      bool req = true;
+      if (cu.t == cu.end) {
+        if (has_next) {
+          cursor_to(nxt);
+          if constexpr (kPaged) take_ids(nxt.t0);
+        }
+        req = has_next && cu.t < cu.end;
+      } else if (kPaged && cu.t - cu.row0 == 64) {
+        take_ids(cu.t);
+        request_ids(has_next, nxt);
+      }
+      Easy e;
+      e.kind = kNone;
+      e.kb = e.vb = nullptr;
+      if (req) {
+        e = issue(stage ^ 1);
+        ++cu.t;
       }
       const uint32_t n_dst = lds_base + (uint32_t)((stage ^ 1) * 2 * TILE_B + wave * NI * 1024);
       const char* s_k = s_kv + stage * 2 * TILE_B;
@@ -768,24 +1033,29 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       // Store steps run only on tiles that hold some of the block's new rows.
       // The rows go out non-temporally: nothing in the launch reads them back
       // (config 3: 40.4 -> 39.6 us per launch).
-      if (fused_store && st_key0 < kb + kKeyTile &&
-          st_key0 + (cur.pos_end - cur.pos0) > kb) {
+      if (fused_store && st_key0 < kb + kKeyTile && st_key0 + nrows / G > kb) {
+        // Pool offset of this lane's row (-1: not stored), computed in the
+        // lane that holds the slot and handed to the lanes that store it.
         const int64_t cap = (int64_t)p.num_blocks * p.block_size;
+        const int64_t slot = p.slot_i64 ? (int64_t)(((uint64_t)st_slot.y << 32) | st_slot.x)
+                                          : (int64_t)(int32_t)st_slot.x;
+        int64_t at = -1;
+        if (slot >= 0 && slot < cap) {
+          const int64_t blk = p.slot_small
+                                  ? (int64_t)fast_div((uint32_t)slot, p.bs_div)
+                                  : slot / p.block_size;
+          at = blk * p.s_blk + (slot - blk * p.block_size) * p.s_slot + cur.h * p.s_head;
+        }
         const int c = lane % CPR;
 #pragma unroll 4
         for (int k = 0; k < NSTEP; ++k) {
           const int holder = k * RPS + lane / CPR;
-          const uint32_t sx = (uint32_t)__shfl((int)st_slot.x, holder, 64);
-          const uint32_t sy = (uint32_t)__shfl((int)st_slot.y, holder, 64);
-          const int64_t slot = p.slot_i64 ? (int64_t)(((uint64_t)sy << 32) | sx)
-                                          : (int64_t)(int32_t)sx;
+          const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)at, holder, 64);
+          const int hi = __shfl((int)(at >> 32), holder, 64);
           const int row = st_base(k) + lane / CPR;
           const int key = st_key0 + row;
-          if (row < BQ && slot >= 0 && slot < cap && key >= kb && key < kb + kKeyTile) {
-            const int64_t blk = p.slot_small ? (int64_t)fast_div((uint32_t)slot, p.bs_div)
-                                             : slot / p.block_size;
-            const int64_t dst = blk * p.s_blk + (slot - blk * p.block_size) * p.s_slot +
-                                cur.h * p.s_head + c * 16;
+          if (row < BQ && hi >= 0 && key >= kb && key < kb + kKeyTile) {
+            const int64_t dst = (int64_t)(((uint64_t)(uint32_t)hi << 32) | lo) + c * 16;
             const int r = key - kb;
             const int off = r * ROWB + ((c ^ swz<D>(r)) << 4);
             st16_nt(p.kp + dst, lds_read16(s_k, off));
@@ -794,138 +1064,156 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
         }
       }
 
-      // ---- S^T = K Q^T for both row tiles ----
-      // K rows of 16-key group kt + 1 are read before group kt's DMA pair:
-      // no LDS read moves across a DMA.
-      static_assert(KT % NI == 0 || NI % KT == 0, "DMA pairs spread evenly over the key groups");
-      constexpr int PAIRS = NI >= KT ? NI / KT : 1;  // DMA pairs after each chosen group
-      constexpr int EVERY = NI >= KT ? 1 : KT / NI;  // every EVERY-th group gets them
-      f32x4_t sacc[2][KT];
-      uint4 ka[2][DS];
+      // On the item's last tile, once its S^T is done, the query rows are
+      // dead: the next item's loads start.  Its store slot goes straight into
+      // st_slot (this item's store steps ran above): a copy at the item's
+      // end would have to wait for the load, and with it for every store
+      // issued after it.
+      auto load_next = [&]() {
+        if (t + 1 == tend && has_next) {
+          load_q(nxt);
+          st_slot = load_slot(nxt);
+        }
+      };
+
+      // One tile on the wave's first NA row tiles.
+      auto reduce = [&](auto NA_) {
+        constexpr int NA = decltype(NA_)::value;
+        // ---- S^T = K Q^T ----
+        // K rows of 16-key group kt + 1 are read before group kt's DMA pair:
+        // no LDS read moves across a DMA.
+        static_assert(KT % NI == 0 || NI % KT == 0, "DMA pairs spread evenly over the key groups");
+        constexpr int PAIRS = NI >= KT ? NI / KT : 1;  // DMA pairs after each chosen group
+        constexpr int EVERY = NI >= KT ? 1 : KT / NI;  // every EVERY-th group gets them
+        // At head_dim 128 the lane's K offsets are rebuilt per tile from opaque
+        // bases: held through the loop they make the compiler spill.
+        int k0 = (g4 ^ kswz) << 4, krow = r16 * ROWB;
+        if constexpr (D > 64) asm volatile("" : "+v"(k0), "+v"(krow));
+        f32x4_t sacc[NA][KT];
+        uint4 ka[2][DS];
 #pragma unroll
-      for (int ds = 0; ds < DS; ++ds)
-        ka[0][ds] = lds_read16(s_k, r16 * ROWB + (((4 * ds + g4) ^ kswz) << 4));
+        for (int ds = 0; ds < DS; ++ds) ka[0][ds] = lds_read16(s_k, krow + (k0 ^ (ds << 6)));
 #pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        if (kt + 1 < KT) {
+        for (int kt = 0; kt < KT; ++kt) {
+          if (kt + 1 < KT) {
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds)
+              ka[(kt + 1) & 1][ds] = lds_read16(s_k, 16 * (kt + 1) * ROWB + krow + (k0 ^ (ds << 6)));
+          }
+#pragma unroll
+          for (int tt = 0; tt < NA; ++tt) sacc[tt][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int ds = 0; ds < DS; ++ds)
-            ka[(kt + 1) & 1][ds] =
-                lds_read16(s_k, (16 * (kt + 1) + r16) * ROWB + (((4 * ds + g4) ^ kswz) << 4));
-        }
-        sacc[0][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        sacc[1][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ds = 0; ds < DS; ++ds) {
-          sacc[0][kt] = M::mfma(ka[kt & 1][ds], qreg[0][ds], sacc[0][kt]);
-          sacc[1][kt] = M::mfma(ka[kt & 1][ds], qreg[1][ds], sacc[1][kt]);
-        }
-        if (spread && kt % EVERY == 0) {
+            for (int tt = 0; tt < NA; ++tt)
+              sacc[tt][kt] = M::mfma(ka[kt & 1][ds], qreg[tt][ds], sacc[tt][kt]);
+          if (kt % EVERY == 0 && (e.kind == kRows || e.kind == kPool)) {
 #pragma unroll
-          for (int j = 0; j < PAIRS; ++j) {
-            const int i = (kt / EVERY) * PAIRS + j;
-            if constexpr (kv_once) {
-              dma16_nt(koff[i], n_kbase, n_dst + i * 1024);
-              dma16_nt(voff[i], n_vbase, n_dst + TILE_B + i * 1024);
-            } else {
-              dma16(koff[i], n_kbase, n_dst + i * 1024);
-              dma16(voff[i], n_vbase, n_dst + TILE_B + i * 1024);
+            for (int j = 0; j < PAIRS; ++j) easy_issue(e, (kt / EVERY) * PAIRS + j, n_dst);
+          }
+          if constexpr (kF8) {
+            if (kt < NIC && e.kind == kCodes) easy_codes(e, kt);
+          }
+        }
+        load_next();
+
+        // V^T goes through a window of DT / 4 operands, the first requested
+        // before the softmax and each later one as an earlier one is used.
+        const int v0 = (((r16 >> 1) & 1) ^ vswz) << 4;
+        const int vrow = (4 * g4 + (r16 >> 2)) * ROWB + ((r16 & 1) << 3);
+        auto read_v = [&](int ks, int dt) -> uint4 {
+          const int off = 32 * ks * ROWB + vrow + (v0 ^ (dt << 5));
+          const uint2 lo = __builtin_bit_cast(uint2, lds_read_tr(s_v, off));
+          const uint2 hi = __builtin_bit_cast(uint2, lds_read_tr(s_v, off + 16 * ROWB));
+          return make_uint4(lo.x, lo.y, hi.x, hi.y);
+        };
+        uint4 vf[DT / 4];
+#pragma unroll
+        for (int dt = 0; dt < DT / 4; ++dt) vf[dt] = read_v(0, dt);
+
+        // ---- online softmax (exp2 domain) and P^T packing ----
+        // Scores stay unscaled until the exponent: p = 2^(s c - m) with
+        // c = scale log2 e > 0 and m the row's running max of s c.  The max
+        // used as reference is raised only when a row's new max exceeds it by
+        // more than kLazy (or on the first scores); in between, p <= 2^kLazy,
+        // which the fp32 sums and 16-bit P hold exactly as well.  Key masking
+        // is applied only on tiles that cross a row's limit.
+        const bool need_mask = kb + kKeyTile > lim_lo;
+        uint4 pb[NA][KS];
+#pragma unroll
+        for (int tt = 0; tt < NA; ++tt) {
+          float sv[KT][4];
+          if (need_mask) {
+            const int rel = lim[tt] - kb - 4 * g4;  // key 16 kt + i of this lane is visible iff < rel
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                sv[kt][i] = 16 * kt + i < rel ? sacc[tt][kt][i] : -INFINITY;
+          } else {
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) sv[kt][i] = sacc[tt][kt][i];
+          }
+          float mx = -INFINITY;
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sv[kt][i]);
+          mx = max_xor16(mx);
+          mx = max_xor32(mx);
+          const float mxs = mx * p.scale_log2;
+          if (__builtin_amdgcn_ballot_w64(mxs > m[tt] + kLazy) != 0) {
+            const float mnew = fmaxf(m[tt], mxs);
+            const float alpha = fast_exp2(m[tt] - mnew);
+            m[tt] = mnew;
+            l[tt] *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[tt][dt] *= alpha;
+          }
+          float pr[KT][4];
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              pr[kt][i] = fast_exp2(fmaf(sv[kt][i], p.scale_log2, -m[tt]));
+              l[tt] += pr[kt][i];
             }
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            pb[tt][ks].x = M::pack2(pr[2 * ks][0], pr[2 * ks][1]);
+            pb[tt][ks].y = M::pack2(pr[2 * ks][2], pr[2 * ks][3]);
+            pb[tt][ks].z = M::pack2(pr[2 * ks + 1][0], pr[2 * ks + 1][1]);
+            pb[tt][ks].w = M::pack2(pr[2 * ks + 1][2], pr[2 * ks + 1][3]);
           }
         }
-      }
-      // The query rows are dead now: on the item's last tile, start the next
-      // item's loads.  Its store slot goes straight into st_slot (this item's
-      // store steps ran at the top of this tile): a copy at the item's end
-      // would have to wait for the load, and with it for every store issued
-      // after it.
-      if (t + 1 == cur.ntiles && has_next) {
-        load_q(nxt);
-        st_slot = load_slot(nxt);
-      }
 
-      // ---- online softmax (exp2 domain) and P^T packing ----
-      // Scores stay unscaled until the exponent: p = 2^(s c - m) with
-      // c = scale log2 e > 0 and m the row's running max of s c.  The max used
-      // as reference is raised only when a row's new max exceeds it by more
-      // than kLazy (or on the first scores); in between, p <= 2^kLazy, which
-      // the fp32 sums and 16-bit P hold exactly as well.  Key masking is
-      // applied only on tiles that cross a row's limit.
-      const bool need_mask = kb + kKeyTile > lim_lo;
-      uint4 pb[2][KS];
+        // ---- O^T += V^T P^T ----
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        float sv[KT][4];
-        if (need_mask) {
-          const int rel = lim[tt] - kb - 4 * g4;  // key 16 kt + i of this lane is visible iff < rel
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-          for (int kt = 0; kt < KT; ++kt)
+          for (int dt = 0; dt < DT; ++dt) {
+            const uint4 a = vf[dt % (DT / 4)];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sv[kt][i] = 16 * kt + i < rel ? sacc[tt][kt][i] : -INFINITY;
-        } else {
-#pragma unroll
-          for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sv[kt][i] = sacc[tt][kt][i];
-        }
-        float mx = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sv[kt][i]);
-        mx = max_xor16(mx);
-        mx = max_xor32(mx);
-        const float mxs = mx * p.scale_log2;
-        if (__builtin_amdgcn_ballot_w64(mxs > m[tt] + kLazy) != 0) {
-          const float mnew = fmaxf(m[tt], mxs);
-          const float alpha = fast_exp2(m[tt] - mnew);
-          m[tt] = mnew;
-          l[tt] *= alpha;
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) o[tt][dt] *= alpha;
-        }
-        float pr[KT][4];
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            pr[kt][i] = fast_exp2(fmaf(sv[kt][i], p.scale_log2, -m[tt]));
-            l[tt] += pr[kt][i];
+            for (int tt = 0; tt < NA; ++tt) o[tt][dt] = M::mfma(a, pb[tt][ks], o[tt][dt]);
+            const int nx = ks * DT + dt + DT / 4;
+            if (nx < KS * DT) vf[dt % (DT / 4)] = read_v(nx / DT, nx % DT);
           }
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          pb[tt][ks].x = M::pack2(pr[2 * ks][0], pr[2 * ks][1]);
-          pb[tt][ks].y = M::pack2(pr[2 * ks][2], pr[2 * ks][3]);
-          pb[tt][ks].z = M::pack2(pr[2 * ks + 1][0], pr[2 * ks + 1][1]);
-          pb[tt][ks].w = M::pack2(pr[2 * ks + 1][2], pr[2 * ks + 1][3]);
-        }
-      }
-
-      // ---- O^T += V^T P^T ----
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const int off = (32 * ks + 4 * g4 + (r16 >> 2)) * ROWB +
-                          (((2 * dt + ((r16 >> 1) & 1)) ^ vswz) << 4) + ((r16 & 1) << 3);
-          const s16x4_t lo = lds_read_tr(s_v, off);
-          const s16x4_t hi = lds_read_tr(s_v, off + 16 * ROWB);
-          uint4 a;
-          a.x = (uint32_t)(uint16_t)lo[0] | ((uint32_t)(uint16_t)lo[1] << 16);
-          a.y = (uint32_t)(uint16_t)lo[2] | ((uint32_t)(uint16_t)lo[3] << 16);
-          a.z = (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16);
-          a.w = (uint32_t)(uint16_t)hi[2] | ((uint32_t)(uint16_t)hi[3] << 16);
-          o[0][dt] = M::mfma(a, pb[0][ks], o[0][dt]);
-          o[1][dt] = M::mfma(a, pb[1][ks], o[1][dt]);
-        }
+      };
+      reduce(std::integral_constant<int, 2>{});
       stage ^= 1;
     }
-    if (cur.ntiles == 0 && has_next) {
+    if (cur.t0 == tend && has_next) {
       // No visible keys in this item: its output is 0 and the next item's
       // loads start here.  `stage` is free: no wave has read it since the
       // last barrier.
-      if (nxt.ntiles > 0)
-        issue_tile(nxt.h, nxt.pool_prefix, nxt.kend, nxt.new_base, nxt.table_row, 0, stage);
+      cursor_to(nxt);
+      if constexpr (kPaged) take_ids(nxt.t0);
+      if (cu.t < cu.end) {
+        issue_now(issue(stage), stage);
+        ++cu.t;
+      }
       load_q(nxt);
       st_slot = load_slot(nxt);
     }
@@ -939,7 +1227,25 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
     // only barrier needed is the one that tells every wave is done reading
     // that stage's K and V.  Chunks are XOR-swizzled by row against bank
     // conflicts.
-    if (cur.ntiles > 0) {
+    if (kSplit && cur.slot >= 0) {
+      // A piece of a split item: unnormalised, in fp32, straight from the
+      // accumulators (64-byte pieces of 16 rows an instruction).
+      const int64_t ps = (int64_t)xcd * kSplitSlots + cur.slot;
+      if (wave == 0) p.part_head[ps] = make_int4(cur.npc, cur.q0 + pos0, nrows, cur.h);
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        const int row = 16 * (wave + 4 * tt) + r16;
+        float lt = l[tt];
+        lt = sum_xor16(lt);
+        lt = sum_xor32(lt);
+        if (row < nrows) {
+          float* const po = p.part_o + (ps * kRowsPerWG + row) * D + 4 * g4;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4_t*>(po + 16 * dt) = o[tt][dt];
+          if (g4 == 0) p.part_ml[ps * kRowsPerWG + row] = make_float2(m[tt], lt);
+        }
+      }
+    } else if (cur.t0 < tend) {
       __syncthreads();
       char* s_o = s_kv + (stage ^ 1) * 2 * TILE_B + wave * 32 * ROWB;
 #pragma unroll
@@ -964,22 +1270,21 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
         const int rw = RPS * j + lane / CPR;  // row within the wave's 32
         const int c = lane % CPR;
         const uint4 v = lds_read16(s_o, rw * ROWB + ((c ^ ((rw % 16) % CPR)) << 4));
-        const int row = 32 * wave + rw;  // MFMA row of the block
-        const int qp = cur.pos0 + row % BQ;
-        if (qp < cur.ql)
-          st16_nt(p.out + (int64_t)(cur.q0 + qp) * p.o_st + (int64_t)(cur.h * G + row / BQ) * p.o_sh +
-                   c * 16,
-               v);
+        const int row = 16 * wave + 64 * (rw / 16) + rw % 16;  // MFMA row of the block
+        if (row < nrows)
+          st16_nt(p.out + (int64_t)(cur.q0 + pos0 + row / G) * p.o_st +
+                      (int64_t)(cur.h * G + row % G) * p.o_sh + c * 16,
+                  v);
       }
     } else {
       // No visible keys: the rows are 0 (the other stage may be receiving the
       // next item's first tile, so nothing is staged).
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) {
-        const int row = 16 * (2 * wave + tt) + r16;
-        const int qp = cur.pos0 + row % BQ;
-        if (qp >= cur.ql) continue;
-        char* dst = p.out + (int64_t)(cur.q0 + qp) * p.o_st + (int64_t)(cur.h * G + row / BQ) * p.o_sh;
+        const int row = 16 * (wave + 4 * tt) + r16;
+        if (row >= nrows) continue;
+        char* dst = p.out + (int64_t)(cur.q0 + pos0 + row / G) * p.o_st +
+                    (int64_t)(cur.h * G + row % G) * p.o_sh;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
           *reinterpret_cast<uint2*>(dst + (16 * dt + 4 * g4) * 2) = make_uint2(0u, 0u);
@@ -990,13 +1295,61 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   }
 }
 
+// Merge of split items' pieces: workgroup (x, y) serves rows 32 y .. 32 y + 31
+// of the item whose first piece is XCD x % 8's piece x / 8 (the XCD that wrote
+// it), and ends at once when there is no such item.
+//   out = sum_j 2^(m_j - M) o_j / sum_j 2^(m_j - M) l_j,  M = max_j m_j.
+template <bool kBF16, int D, int G>
+__global__ __launch_bounds__(256) void varlen_merge_kernel(VarlenParams p) {
+  constexpr int LPR = D / 4;       // lanes per row, four outputs each
+  constexpr int RPP = 256 / LPR;   // rows per pass
+  const int xcd = (int)blockIdx.x % kXcds, slot = (int)blockIdx.x / kXcds;
+  const int64_t ps = (int64_t)xcd * kSplitSlots + slot;
+  const int count = p.part_count[xcd];
+  const int4 hd = p.part_head[ps];  // read whether or not it was written
+  const int row0 = (int)blockIdx.y * 32;
+  if (slot >= count || hd.x == 0 || row0 >= hd.z) return;
+  const int col = threadIdx.x % LPR;
+  for (int row = row0 + threadIdx.x / LPR; row < min(row0 + 32, hd.z); row += RPP) {
+    const float* po = p.part_o + (ps * kRowsPerWG + row) * D + 4 * col;
+    const float2* pm = p.part_ml + ps * kRowsPerWG + row;
+    float M = -1.0e30f, L = 0.f;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    for (int j0 = 0; j0 < hd.x; j0 += 4) {
+      f32x4_t oj[4];
+      float2 ml[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t at = min(j0 + j, hd.x - 1) * (int64_t)kRowsPerWG;
+        ml[j] = pm[at];
+        oj[j] = *reinterpret_cast<const f32x4_t*>(po + at * D);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j0 + j >= hd.x) break;
+        const float mn = fmaxf(M, ml[j].x);
+        const float a = fast_exp2(M - mn), b = fast_exp2(ml[j].x - mn);
+        acc = acc * a + oj[j] * b;
+        L = L * a + ml[j].y * b;
+        M = mn;
+      }
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    uint2 w;
+    w.x = Mma<kBF16>::pack2(acc[0] * inv, acc[1] * inv);
+    w.y = Mma<kBF16>::pack2(acc[2] * inv, acc[3] * inv);
+    *reinterpret_cast<uint2*>(p.out + (int64_t)(hd.y + row / G) * p.o_st +
+                              (int64_t)(hd.w * G + row % G) * p.o_sh + col * 8) = w;
+  }
+}
+
 // Launch the persistent grid: per XCD, as many workgroups as the kernel
 // keeps resident on one XCD's CUs, or fewer when the XCD's item list (at
 // most items_per_xcd long) is shorter.
-template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce = false,
-          bool kF8 = false, bool kPro = false>
-static void launch_persistent(const VarlenParams& p, int64_t items_per_xcd, hipStream_t st) {
-  const auto kern = varlen_attention_kernel<kBF16, D, G, kCausal, kPaged, kOnce, kF8, kPro>;
+template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce, bool kF8, bool kPro,
+          bool kSplit>
+static void launch_grid(const VarlenParams& p, int64_t items_per_xcd, hipStream_t st) {
+  const auto kern = varlen_attention_kernel<kBF16, D, G, kCausal, kPaged, kOnce, kF8, kPro, kSplit>;
   // Resident workgroups per CU, queried once (a failed query is not cached:
   // the launch then assumes 1, which is correct but leaves slots idle).
   static std::atomic<int> cached{0};
@@ -1014,9 +1367,22 @@ static void launch_persistent(const VarlenParams& p, int64_t items_per_xcd, hipS
   int64_t cus_per_xcd = current_device_cus() / kXcds;
   if (cus_per_xcd < 1) cus_per_xcd = 1;
   int64_t per_xcd = (int64_t)per_cu * cus_per_xcd;
-  if (per_xcd > items_per_xcd) per_xcd = items_per_xcd;
+  if (per_xcd > items_per_xcd && !kSplit) per_xcd = items_per_xcd;
   if (per_xcd < 1) per_xcd = 1;
   hipLaunchKernelGGL(kern, dim3((unsigned)(per_xcd * kXcds)), dim3(kVarlenThreads), 0, st, p);
+  if constexpr (kSplit)
+    hipLaunchKernelGGL((varlen_merge_kernel<kBF16, D, G>), dim3(kSplitSlots * kXcds, 4), dim3(256),
+                       0, st, p);
+}
+
+template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce = false,
+          bool kF8 = false, bool kPro = false>
+static void launch_persistent(const VarlenParams& p, int64_t items_per_xcd, hipStream_t st) {
+  if constexpr (!kOnce) {
+    if (p.split)
+      return launch_grid<kBF16, D, G, kCausal, kPaged, false, kF8, kPro, true>(p, items_per_xcd, st);
+  }
+  launch_grid<kBF16, D, G, kCausal, kPaged, kOnce, kF8, kPro, false>(p, items_per_xcd, st);
 }
 
 template <bool kBF16, int D, int G, bool kCausal>

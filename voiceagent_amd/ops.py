@@ -376,7 +376,8 @@ def _fast_calls():
                 return ctypes.cast(fn, ctypes.c_void_p).value
 
             mod.set_entries(addr(lib.va_paged_decode), addr(lib.va_paged_decode_workspace_bytes),
-                            addr(lib.va_varlen_attention), addr(lib.va_store_kvcache),
+                            addr(lib.va_varlen_attention),
+                            addr(lib.va_varlen_split_workspace_bytes), addr(lib.va_store_kvcache),
                             addr(lib.va_qk_norm_rope))
             _FAST = mod
     return _FAST
@@ -746,6 +747,18 @@ def varlen_attention(
     lib = N.lib()
     index = _device_index(device)
     with _current(index):
+        nbytes = lib.va_varlen_split_workspace_bytes(ctypes.byref(args))
+        if nbytes:
+            # A tensor of this call alone: torch's allocator hands its memory
+            # out again in the order of this stream (or of the captured graph).
+            # Without it the launch runs unsplit, as it also does when memory
+            # is short.
+            try:
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+                args.workspace = ws.data_ptr()
+                args.workspace_bytes = nbytes
+            except torch.OutOfMemoryError:
+                pass
         N.check("va_varlen_attention",
                 lib.va_varlen_attention(ctypes.byref(args), _raw_stream(index)))
     return out
