@@ -55,8 +55,8 @@ HIPCC_FLAGS = [
 # accumulators is VALU work, and AGPR accumulators would be copied out and
 # back on every tile.
 EXTRA_FLAGS = {
-    "paged_decode_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
-    "paged_decode_f16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
+    f"paged_decode_{unit}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"]
+    for unit in ("bf16", "f16", "bf16_f8", "f16_f8")
 }
 
 

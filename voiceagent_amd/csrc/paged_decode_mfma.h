@@ -225,7 +225,7 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
   const int h = blockIdx.x;
   const int part = blockIdx.z;
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: tile addresses stay scalar
   const int lane = tid & 63;
   const int r16 = lane & 15;   // MFMA row / column index of this lane
   const int c4 = lane >> 4;    // MFMA k-group of this lane
@@ -243,6 +243,13 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
   // Block of the wave's tile `lane` (tile 64 i + lane after refills): `tab`
   // serves the DMA issue, which runs S tiles ahead; `tab_proc` is the copy
   // the tile being reduced reads (refreshed when it reaches the refill).
+  // A tile's address was formed from a wave index the compiler took for
+  // divergent: ~60 of a tile's ~200 vector operations.  With `wave` uniform it
+  // is scalar work, and over 16-bit pools the offsets of the tiles issued
+  // from the loop come from `toff`, formed 64 at a time, a lane each (kNoRow
+  // for a block id outside the pool).  Batch 32 x U[60,600] with the prologue:
+  // 13.7 -> 13.3 us a layer; 128 over FP8 pools: 27.1 -> 24.9 (26.6 with
+  // `toff`, whose readlanes an FP8 tile's shorter loop does not hide).
   const uint32_t* const tabw = reinterpret_cast<const uint32_t*>(p.table);
   auto block_of = [&](int tok) -> int {  // table entry of token tok's block, 0 past the width
     const int idx = (int)fast_div((uint32_t)tok, p.bs_div);
@@ -359,25 +366,23 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
   }
   const char* zero_row = reinterpret_cast<const char*>(&kDecZeroRow);
   const int64_t head_off = (int64_t)h * p.s_head;
+  constexpr int64_t kNoRow = INT64_MIN;
+  auto row_off = [&](int tok, int blk) -> int64_t {
+    return blk >= 0 && blk < p.num_blocks
+               ? (int64_t)blk * p.s_blk +
+                     (int64_t)fast_mod((uint32_t)tok, p.bs_div) * p.s_slot + head_off
+               : kNoRow;
+  };
+  auto tile_off = [&](int64_t offs, int k) -> int64_t {  // lane k % 64's entry
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)offs, k & 63);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(offs >> 32), k & 63);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+  };
+  int64_t toff = kNoRow;
   int span = 0;  // tokens of this partition (set once the length is known)
-  // Issue tile k of this wave into stage k % S.  Tiles whose block id is
-  // outside [0, num_blocks) read zeros (their scores are masked).
-  auto issue = [&](int k) {
-    if (k > 0 && (k & 63) == 0) {
-      // Next 64 tiles of this wave: refill the block-id prefetch.
-      const int c = wave + W * (k + lane);
-      tab = c * kChunk < span ? block_of(start + c * kChunk) : 0;
-      if (has_mask) {
-        mask_load(start + c * kChunk);
-        mbits = mask_bits();
-      }
-    }
-    const int tb = start + (wave + W * k) * kChunk;
-    const int32_t blk = __builtin_amdgcn_readlane(tab, k & 63);
+  auto issue_at = [&](int k, int64_t off) {
     const uint32_t dst = lds_wave + (uint32_t)((k % S) * STAGE_B);
-    if (blk >= 0 && blk < p.num_blocks) {
-      const int64_t off = (int64_t)blk * p.s_blk + (int64_t)fast_mod((uint32_t)tb, p.bs_div) * p.s_slot +
-                          head_off;
+    if (off != kNoRow) {
       const char* kb = uniform_ptr(p.kp + off);
       const char* vb = uniform_ptr(p.vp + off);
 #pragma unroll
@@ -388,6 +393,28 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
 #pragma unroll
       for (int i = 0; i < 2 * NI; ++i) dma16(zero_row, dst + i * 1024);
     }
+  };
+  // Issue tile k of this wave into stage k % S.  Tiles whose block id is
+  // outside [0, num_blocks) read zeros (their scores are masked).
+  auto issue = [&](int k) {
+    if (k > 0 && (k & 63) == 0) {
+      // Next 64 tiles of this wave: refill the block-id prefetch.
+      const int c = wave + W * (k + lane);
+      tab = c * kChunk < span ? block_of(start + c * kChunk) : 0;
+      if constexpr (!kF8) toff = row_off(start + c * kChunk, tab);
+      if (has_mask) {
+        mask_load(start + c * kChunk);
+        mbits = mask_bits();
+      }
+    }
+    if constexpr (kF8)
+      issue_at(k, row_off(start + (wave + W * k) * kChunk, __builtin_amdgcn_readlane(tab, k & 63)));
+    else
+      issue_at(k, tile_off(toff, k));
+  };
+  // The wave's first tiles, before the offsets of all 64 are formed.
+  auto issue_first = [&](int k) {
+    issue_at(k, row_off(start + (wave + W * k) * kChunk, __builtin_amdgcn_readlane(tab, k)));
   };
 
   // With fixed partitions (one per pair, the common decode batch, or a split
@@ -418,7 +445,7 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
     // past it.  The last partition also takes any tokens past its P, so it
     // requests all of its first tiles.
     for (int k = 0; k < S; ++k)
-      if (part == p.max_parts - 1 || (wave + W * k) * kChunk < P) issue(k);
+      if (part == p.max_parts - 1 || (wave + W * k) * kChunk < P) issue_first(k);
   }
   if constexpr (kProlog) load_rotary<E, LPR>(p.pro, pos, col, D, pro_c, pro_s);
 
@@ -524,12 +551,13 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
 
   if (!early) {
     for (int k = 0; k < S; ++k)
-      if (k < ntw) issue(k);
+      if (k < ntw) issue_first(k);
     // The partition's start follows from the length here, so the mask words
     // are requested behind the first tiles.
     if (has_mask) mask_load(start + (wave + W * lane) * kChunk);
   }
   if (has_mask) mbits = mask_bits();
+  if (!kF8 && ntw > S) toff = row_off(start + (wave + W * lane) * kChunk, tab);
   int tab_proc = tab;
   uint32_t mbits_proc = mbits;
 
@@ -537,11 +565,11 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
   mf_f32x4 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
-  // Pool offset of this lane's 16 bytes of the current row (-1: none).  The
+  // Pool offset of this lane's 16 bytes of the current row (kNoRow: none).  The
   // row is written after the last workgroup barrier: a barrier waits for
   // every store the wave has in flight, so a write issued in the loop would
   // hold up the merge below by a whole HBM write round trip.
-  int64_t cur_dst = -1;
+  int64_t cur_dst = kNoRow;
   const int kswz = dec_swz<D>(r16);
   const int vrow = 4 * c4 + (r16 >> 2);
   const int vswz = dec_swz<D>(vrow);
@@ -564,12 +592,17 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
 
     if (c == new_tile) {
       // The current row: put it in place of the staged pool row, and note
-      // its slot (new_slots[b], or the table slot of L - 1) for the pool
-      // write at the end.
-      int64_t slot = new_slot;
-      if (p.new_slots == nullptr)
-        slot = blk_ok ? (int64_t)blk * p.block_size + fast_mod((uint32_t)new_tok, p.bs_div) : -1;
-      if (slot >= 0 && slot < cap && rg == 0) {
+      // its pool offset (of new_slots[b], or of the tile's own row) for the
+      // pool write at the end.
+      int64_t at = kNoRow;
+      if (p.new_slots == nullptr) {
+        if (blk_ok) at = row_off(new_tok, blk);
+      } else if (new_slot >= 0 && new_slot < cap) {
+        const int64_t sb = p.slot_small ? (int64_t)fast_div((uint32_t)new_slot, p.bs_div)
+                                        : new_slot / p.block_size;
+        at = sb * p.s_blk + (new_slot - sb * p.block_size) * p.s_slot + head_off;
+      }
+      if (at != kNoRow && rg == 0) {
         const int r = new_tok - tb;
         const int pos16 = (col ^ dec_swz<D>(r)) << 4;
         if constexpr (kF8) {  // the lane's eight codes, in the stages' layout
@@ -580,10 +613,7 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
           *reinterpret_cast<uint4*>(sK + r * ROWB + pos16) = kcur;
           *reinterpret_cast<uint4*>(sV + r * ROWB + pos16) = vcur;
         }
-        const int64_t sb = p.slot_small ? (int64_t)fast_div((uint32_t)slot, p.bs_div)
-                                        : slot / p.block_size;
-        cur_dst = sb * p.s_blk + (slot - sb * p.block_size) * p.s_slot + head_off +
-                  col * (kF8 ? 8 : 16);
+        cur_dst = at + col * (kF8 ? 8 : 16);
       }
     }
 
@@ -758,7 +788,7 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
       }
     }
   }
-  if (cur_dst >= 0) {
+  if (cur_dst != kNoRow) {
     if constexpr (kF8) {
       *reinterpret_cast<uint2*>(p.kp + cur_dst) = kq;
       *reinterpret_cast<uint2*>(p.vp + cur_dst) = vq;
