@@ -54,26 +54,63 @@ static SplitLayout split_layout(int head_dim) {
 // (9 prompts of 60-594 tokens and 24 decoding sequences beside three prompts
 // of 530, which this leaves whole, lost 2.5-3.4 us to a merge launch with
 // nothing to merge.)
+// Per XCD: slots, the items with `rows` MFMA rows each, and the tiles of the
+// longest item.
+struct VarlenLoad {
+  int64_t slots, items, longest;
+};
+static VarlenLoad varlen_load(const va_varlen_args* a, int rows) {
+  const int BQ = rows * a->num_kv_heads / a->num_heads;
+  const int64_t table_keys =
+      a->pool.k != nullptr ? (int64_t)a->table_width * a->pool.block_size : 0;
+  const int64_t keys = a->max_seqlen_q > table_keys ? a->max_seqlen_q : table_keys;
+  VarlenLoad w;
+  w.slots = 2 * (int64_t)current_device_cus() / kXcds;
+  w.items = (a->num_kv_heads * ((int64_t)a->total_q / BQ + a->num_seqs) + kXcds - 1) / kXcds;
+  w.longest = (keys + kKeyTile - 1) / kKeyTile;
+  return w;
+}
+
+// Tiles of a piece the device would choose (plan_split).
+static int64_t split_piece(const VarlenLoad& w) {
+  const int64_t over =
+      std::min<int64_t>(std::max(w.slots - w.items / 4, (w.slots + 1) / 2), kSplitSlots / 2);
+  return std::max<int64_t>(w.items * w.longest / 2 / over, kSplitMinTiles);
+}
+
 static bool split_wanted(const va_varlen_args* a) {
   if (a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0) return false;
   const int G = a->num_heads / a->num_kv_heads;
   if (G != 1 && G != 2 && G != 4 && G != 8) return false;
   if (a->head_dim != 64 && a->head_dim != 128) return false;
   if (a->num_seqs <= 0 || a->total_q <= 0) return false;
-  const int BQ = kRowsPerWG / G;
-  if (!a->causal && a->pool.k == nullptr && a->max_seqlen_q <= BQ) return false;  // kOnce
+  if (!a->causal && a->pool.k == nullptr && a->max_seqlen_q <= kRowsPerWG / G) return false;  // kOnce
   const int64_t pairs = (int64_t)a->num_seqs * a->num_kv_heads;
   if ((pairs + kXcds - 1) / kXcds > 64) return false;  // the plan holds a pair per lane
-  const int64_t table_keys =
-      a->pool.k != nullptr ? (int64_t)a->table_width * a->pool.block_size : 0;
-  const int64_t keys = a->max_seqlen_q > table_keys ? a->max_seqlen_q : table_keys;
-  const int64_t longest = (keys + kKeyTile - 1) / kKeyTile;
-  const int64_t slots = 2 * (int64_t)current_device_cus() / kXcds;  // of one XCD
-  const int64_t items =
-      (a->num_kv_heads * ((int64_t)a->total_q / BQ + a->num_seqs) + kXcds - 1) / kXcds;
-  const int64_t over = std::min<int64_t>(std::max(slots - items / 4, (slots + 1) / 2), kSplitSlots / 2);
-  const int64_t piece = std::max<int64_t>(items * longest / 2 / over, kSplitMinTiles);
-  return longest >= piece + piece / 4 + 5;
+  const VarlenLoad w = varlen_load(a, kRowsPerWG);
+  const int64_t piece = split_piece(w);
+  return w.longest >= piece + piece / 4 + 5;
+}
+
+// Whether a causal launch takes items of 64 rows (kHalf).  The last slot to
+// end has about max(longest item, tiles / slots) tiles (a piece when split);
+// with 64 rows an item's tile takes 0.6-0.7 of the time, and there are up to
+// twice the items, whose set-up and staging cost more than that once they
+// come in more than two rounds.  So short blocks (decoding sequences, chunks
+// of a few tokens) and launches that do not fill the slots take them; a full
+// launch of prompts, or long prefixes over enough rows to fill the slots, do
+// not.  128 against 64 rows, us with the prologue: one prompt of 420 tokens
+// 24.5 / 23.4; 26 decoding sequences with 3 short prompts 21.3 / 18.7; chunks
+// of a few tokens over long prefixes 61.8 / 40.7; 9 prompts of 60-594 tokens
+// 39.2 / 37.2; 16 prompts of 109-439 (three rounds of half items) 39.8 / 45.8.
+static bool half_rows_wanted(const va_varlen_args* a, bool split) {
+  if (!a->causal || a->prologue != nullptr) return false;
+  const VarlenLoad full = varlen_load(a, kRowsPerWG), half = varlen_load(a, kRowsPerWG / 2);
+  auto tiles = [&](const VarlenLoad& w) {
+    const int64_t share = (w.items * w.longest / 2 + w.slots - 1) / w.slots;
+    return std::max(split ? split_piece(w) : w.longest, share);
+  };
+  return half.items <= 2 * half.slots && tiles(half) * 7 < tiles(full) * 10;
 }
 
 }  // namespace va
@@ -186,7 +223,10 @@ int va::varlen_native(const va_varlen_args* a, void* stream) {
               a->head_dim, G);
     return VA_ERR_UNSUPPORTED;
   }
-  const int BQ = kRowsPerWG / G;
+  const bool split = a->workspace != nullptr && (uintptr_t)a->workspace % 16 == 0 &&
+                     split_wanted(a) && a->workspace_bytes >= split_layout(a->head_dim).total;
+  const bool half = half_rows_wanted(a, split);
+  const int BQ = (half ? kRowsPerWG / 2 : kRowsPerWG) / G;
   const int nqb = (a->max_seqlen_q + BQ - 1) / BQ;
   if (nqb == 0) return VA_OK;
   VA_CHECK_ARG(nqb <= 65535 * 16, "va_varlen_attention: max_seqlen_q too large");
@@ -263,21 +303,19 @@ int va::varlen_native(const va_varlen_args* a, void* stream) {
   p.block16 = has_pool && p.block_size % 16 == 0 && p.s_slot >= 0 &&
               15 * p.s_slot + a->head_dim * kv_eb < ((int64_t)1 << 31);
 
-  p.split = 0;
+  p.half = half;
+  p.split = split;
   p.part_o = nullptr;
   p.part_ml = nullptr;
   p.part_head = nullptr;
   p.part_count = nullptr;
-  if (a->workspace != nullptr && (uintptr_t)a->workspace % 16 == 0 && split_wanted(a)) {
+  if (split) {
     const SplitLayout l = split_layout(a->head_dim);
-    if (a->workspace_bytes >= l.total) {
-      char* const ws = (char*)a->workspace;
-      p.split = 1;
-      p.part_o = (float*)(ws + l.o);
-      p.part_ml = (float2*)(ws + l.ml);
-      p.part_head = (int4*)(ws + l.head);
-      p.part_count = (int32_t*)(ws + l.count);
-    }
+    char* const ws = (char*)a->workspace;
+    p.part_o = (float*)(ws + l.o);
+    p.part_ml = (float2*)(ws + l.ml);
+    p.part_head = (int4*)(ws + l.head);
+    p.part_count = (int32_t*)(ws + l.count);
   }
 
   // Persistent 1-D grid over kXcds interleaved item lists; see the kernel.

@@ -91,6 +91,7 @@ struct VarlenParams {
   // Split items (kSplit; all null / 0 without a workspace): per XCD
   // kSplitSlots pieces, their (m, l) and o, what they belong to, how many.
   int32_t split;  // host: take the kSplit instantiation
+  int32_t half;   // host: take the kHalf instantiation
   float* part_o;
   float2* part_ml;
   int4* part_head;
@@ -219,10 +220,17 @@ __device__ inline s16x4_t lds_read_tr(const char* base, int off) {
 // kSplit: the launch has a workspace and may split items (an instantiation of
 // its own: the plan's state costs the others scalar registers, 1 us of 41 on
 // a launch of 32 prompts).
+//
+// kHalf: 64 MFMA rows per item, one 16-row tile per wave.  A tile's body is
+// bound by the wave's own chain (S^T, softmax, O^T; ~2 us with two row tiles,
+// ~1.2 with one, alone on a CU), so a launch that leaves slots idle, or whose
+// blocks are short anyway, ends sooner on items of half the rows (the host's
+// rule: half_rows_wanted).
 template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce, bool kF8, bool kPro,
-          bool kSplit>
+          bool kSplit, bool kHalf>
 __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(VarlenParams p) {
-  constexpr int BQ = kRowsPerWG / G;       // query positions per workgroup
+  constexpr int NR = kHalf ? 1 : 2;        // 16-row tiles per wave
+  constexpr int BQ = 64 * NR / G;          // query positions per workgroup
   constexpr int DS = D / 32;               // k-steps of the S^T MFMA
   constexpr int DT = D / 16;               // 16-wide d tiles of O^T
   constexpr int ROWB = D * 2;              // bytes per K/V row
@@ -232,7 +240,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   constexpr int NI = TILE_B / 1024 / 4;    // DMA instructions per wave per tile, K or V
   constexpr int KT = kKeyTile / 16;        // 16-key tiles per key tile
   constexpr int KS = kKeyTile / 32;        // 32-key MFMA steps per key tile
-  static_assert(BQ % 16 == 0, "query block must hold whole 16-row tiles");
+  static_assert(!kHalf || !kPro, "the query prologue takes two row tiles");
   static_assert(NI * 4 * 1024 == TILE_B, "tile DMA split");
   using M = Mma<kBF16>;
 
@@ -749,13 +757,13 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   // ---- query rows and store slots of an item ----
   // Two 16-row tiles per wave: row 16 (wave + 4 tt) + r16 of the block is
   // query position pos0 + row / G of head h G + row % G.
-  uint4 qreg[2][DS];
+  uint4 qreg[NR][DS];
   // kPro: the rotary position of each of the lane's two query rows (the row
   // of the item's last query for rows past the end, whose output is unused).
   int64_t qrot[2] = {0, 0};
   auto load_q = [&](const Item& it) {
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
+    for (int tt = 0; tt < NR; ++tt) {
       const int row = 16 * (wave + 4 * tt) + r16;
       const int qpos = it.qb * BQ + row / G;
       const int qhead = it.h * G + row % G;
@@ -833,9 +841,9 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
     const int prefix = prefix_of(cur);
     const int kend = kend_of(cur);
     const int tend = cur.t1;
-    int lim[2];
+    int lim[NR];
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
+    for (int tt = 0; tt < NR; ++tt) {
       // Visible keys per row: j < lim[tt].  Rows past the end of the
       // sequence have zero queries; their outputs are never written.
       const int qpos = pos0 + (16 * (wave + 4 * tt) + r16) / G;
@@ -846,14 +854,18 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
     const int lim_lo = kCausal ? min(kend, cur.kl - cur.ql + pos0 + 16 * wave / G + 1) : kend;
     const int st_key0 = prefix + pos0;  // key of the block's first row
 
-    float m[2] = {-1.0e30f, -1.0e30f};
-    float l[2] = {0.f, 0.f};
-    f32x4_t o[2][DT];
+    float m[NR], l[NR];
+    f32x4_t o[NR][DT];
+#pragma unroll
+    for (int tt = 0; tt < NR; ++tt) {
+      m[tt] = -1.0e30f;
+      l[tt] = 0.f;
+    }
     // With the query prologue the accumulators are zeroed after it, at the
     // item's first tile, so they hold no registers while it runs.
     if constexpr (!kPro) {
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
+      for (int tt = 0; tt < NR; ++tt)
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[tt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
@@ -871,7 +883,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       // make the compiler's own wait for them fall here, before the next
       // DMA, where it is free (a later wait would also stall on that DMA).
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
+      for (int tt = 0; tt < NR; ++tt)
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds)
           asm volatile("" ::"v"(qreg[tt][ds].x), "v"(qreg[tt][ds].y), "v"(qreg[tt][ds].z),
@@ -1201,7 +1213,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
             if (nx < KS * DT) vf[dt % (DT / 4)] = read_v(nx / DT, nx % DT);
           }
       };
-      reduce(std::integral_constant<int, 2>{});
+      reduce(std::integral_constant<int, NR>{});
       stage ^= 1;
     }
     if (cur.t0 == tend && has_next) {
@@ -1223,7 +1235,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
     // rows (16 bytes per lane, CPR lanes per row) instead of 8-byte pieces of
     // 16 rows: the narrow pattern cost more per byte.  The staging area is
     // the stage of the item's last tile (the next item's first tile is
-    // landing in the other one); wave w uses its own 32 rows of it, so the
+    // landing in the other one); wave w uses its own 16 NR rows of it, so the
     // only barrier needed is the one that tells every wave is done reading
     // that stage's K and V.  Chunks are XOR-swizzled by row against bank
     // conflicts.
@@ -1233,7 +1245,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       const int64_t ps = (int64_t)xcd * kSplitSlots + cur.slot;
       if (wave == 0) p.part_head[ps] = make_int4(cur.npc, cur.q0 + pos0, nrows, cur.h);
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
+      for (int tt = 0; tt < NR; ++tt) {
         const int row = 16 * (wave + 4 * tt) + r16;
         float lt = l[tt];
         lt = sum_xor16(lt);
@@ -1247,9 +1259,9 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       }
     } else if (cur.t0 < tend) {
       __syncthreads();
-      char* s_o = s_kv + (stage ^ 1) * 2 * TILE_B + wave * 32 * ROWB;
+      char* s_o = s_kv + (stage ^ 1) * 2 * TILE_B + wave * 16 * NR * ROWB;
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
+      for (int tt = 0; tt < NR; ++tt) {
         float lt = l[tt];
         lt = sum_xor16(lt);
         lt = sum_xor32(lt);
@@ -1266,8 +1278,8 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       __builtin_amdgcn_wave_barrier();
       constexpr int RPS = 64 / CPR;  // rows per store instruction
 #pragma unroll 2
-      for (int j = 0; j < 32 / RPS; ++j) {
-        const int rw = RPS * j + lane / CPR;  // row within the wave's 32
+      for (int j = 0; j < 16 * NR / RPS; ++j) {
+        const int rw = RPS * j + lane / CPR;  // row within the wave's 16 NR
         const int c = lane % CPR;
         const uint4 v = lds_read16(s_o, rw * ROWB + ((c ^ ((rw % 16) % CPR)) << 4));
         const int row = 16 * wave + 64 * (rw / 16) + rw % 16;  // MFMA row of the block
@@ -1280,7 +1292,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       // No visible keys: the rows are 0 (the other stage may be receiving the
       // next item's first tile, so nothing is staged).
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
+      for (int tt = 0; tt < NR; ++tt) {
         const int row = 16 * (wave + 4 * tt) + r16;
         if (row >= nrows) continue;
         char* dst = p.out + (int64_t)(cur.q0 + pos0 + row / G) * p.o_st +
@@ -1347,9 +1359,9 @@ __global__ __launch_bounds__(256) void varlen_merge_kernel(VarlenParams p) {
 // keeps resident on one XCD's CUs, or fewer when the XCD's item list (at
 // most items_per_xcd long) is shorter.
 template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce, bool kF8, bool kPro,
-          bool kSplit>
+          bool kSplit, bool kHalf>
 static void launch_grid(const VarlenParams& p, int64_t items_per_xcd, hipStream_t st) {
-  const auto kern = varlen_attention_kernel<kBF16, D, G, kCausal, kPaged, kOnce, kF8, kPro, kSplit>;
+  const auto kern = varlen_attention_kernel<kBF16, D, G, kCausal, kPaged, kOnce, kF8, kPro, kSplit, kHalf>;
   // Resident workgroups per CU, queried once (a failed query is not cached:
   // the launch then assumes 1, which is correct but leaves slots idle).
   static std::atomic<int> cached{0};
@@ -1378,11 +1390,19 @@ static void launch_grid(const VarlenParams& p, int64_t items_per_xcd, hipStream_
 template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce = false,
           bool kF8 = false, bool kPro = false>
 static void launch_persistent(const VarlenParams& p, int64_t items_per_xcd, hipStream_t st) {
+  if constexpr (kCausal && !kPro) {
+    if (p.half)
+      return p.split ? launch_grid<kBF16, D, G, true, kPaged, false, kF8, false, true, true>(
+                           p, items_per_xcd, st)
+                     : launch_grid<kBF16, D, G, true, kPaged, false, kF8, false, false, true>(
+                           p, items_per_xcd, st);
+  }
   if constexpr (!kOnce) {
     if (p.split)
-      return launch_grid<kBF16, D, G, kCausal, kPaged, false, kF8, kPro, true>(p, items_per_xcd, st);
+      return launch_grid<kBF16, D, G, kCausal, kPaged, false, kF8, kPro, true, false>(
+          p, items_per_xcd, st);
   }
-  launch_grid<kBF16, D, G, kCausal, kPaged, kOnce, kF8, kPro, false>(p, items_per_xcd, st);
+  launch_grid<kBF16, D, G, kCausal, kPaged, kOnce, kF8, kPro, false, false>(p, items_per_xcd, st);
 }
 
 template <bool kBF16, int D, int G, bool kCausal>
