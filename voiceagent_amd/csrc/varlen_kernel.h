@@ -14,9 +14,8 @@
 // (sequence, kv head, query block) with all G query heads of the kv group,
 // so its 128 MFMA rows are BQ = 128 / G query positions x G heads, row
 // r = position G + head: a short block fills the first rows only.  Wave w
-// owns the 16-row tiles w and w + 4 and leaves out those past the block's
-// last row, so a decoding sequence in a mixed batch (G rows) costs one tile
-// of one wave.  Workgroups are persistent: the grid fills the
+// owns the 16-row tiles w and w + 4 (items of 64 rows, kHalf: tile w).
+// Workgroups are persistent: the grid fills the
 // GPU's workgroup slots once and each workgroup works through a list of
 // items.  Keys stream through LDS in 64-key tiles (K and V row-major,
 // 16-byte chunks XOR-swizzled by row against bank conflicts) over a ring of
