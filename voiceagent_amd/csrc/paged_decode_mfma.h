@@ -429,7 +429,14 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
   // rotary rows depend on the position and are requested after the DMA, so
   // the prologue arithmetic waits for the early tiles anyway, which it
   // precedes only by a few hundred cycles.
+  // Without the prologue the block ids are waited for on every path before any
+  // DMA, here and where they are read again below: a wait left to the first use
+  // after the tiles' DMA (`toff`, the loop's readlanes) waits for those tiles
+  // too.  One context of 16384 tokens: 16.3 -> 15.9 us (exact length), 17.4 ->
+  // 16.8 (a bound).  With the prologue, whose arithmetic then runs behind the
+  // second ids' round trip, 32 sequences lost 1%: there the ids stay pending.
   const bool early = !p.dyn_split;
+  if constexpr (!kProlog) asm volatile("" ::"v"(tab));
   if (early) {
     if constexpr (!kProlog) {
 #pragma unroll
@@ -477,6 +484,7 @@ __global__ __launch_bounds__((MfmaWaves<D, kWaves>::W * 64), 1) void paged_decod
     if (start < L) {
       const int c = wave + W * lane;
       tab = c * kChunk < P ? block_of(start + c * kChunk) : 0;
+      if constexpr (!kProlog) asm volatile("" ::"v"(tab));
     }
   }
   if (start >= L) {
