@@ -203,6 +203,14 @@ __device__ inline s16x4_t lds_read_tr(const char* base, int off) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(base + off));
 }
 
+// Workgroups the registers leave room for per CU (one wave of each per SIMD).
+// head_dim 64 was left to what the compiler happened to use: at 169-172 VGPRs
+// the paged kernels of groups 4 and 8 fell from three workgroups to two (32
+// prompts of 50-450 tokens, 32/8 heads: 38.2 us with two, 34.0 with three and
+// a few registers spilled), and 64-row items at 129-134 from four to three (28
+// decoding sequences with 4 prompts, 32/8 heads: 27.7 us, 19.5 with four).
+constexpr int waves_per_simd(int d, bool half) { return d == 64 ? (half ? 4 : 3) : 2; }
+
 // kPaged: keys j < k_len - q_len come from the pool through the block table
 // (launches with a pool); otherwise every key comes from k/v.  kF8 (with
 // kPaged): the pool holds OCP e4m3 codes.  A tile's pool rows are copied as
@@ -227,7 +235,8 @@ __device__ inline s16x4_t lds_read_tr(const char* base, int off) {
 // rule: half_rows_wanted).
 template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce, bool kF8, bool kPro,
           bool kSplit, bool kHalf>
-__global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(VarlenParams p) {
+__global__ __launch_bounds__(kVarlenThreads, waves_per_simd(D, kHalf)) void
+varlen_attention_kernel(VarlenParams p) {
   constexpr int NR = kHalf ? 1 : 2;        // 16-row tiles per wave
   constexpr int BQ = 64 * NR / G;          // query positions per workgroup
   constexpr int DS = D / 32;               // k-steps of the S^T MFMA
@@ -482,22 +491,31 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   // row RPI i + l / CPR of them, chunk position l % CPR, so it reads logical
   // chunk (l % CPR) ^ swz(row) of that key.
   static_assert(NI * RPI == 16, "a wave stages 16 rows of a tile");
-  uint32_t koff[NI], voff[NI];  // per-lane byte offsets inside the wave's 16 k/v rows
+  // The offsets are those of k/v rows, or (off_pool) of 16 pool rows of one
+  // block: a launch changes over once or twice an item, so the tile loop holds
+  // one set and has one form of request.
+  uint32_t koff[NI], voff[NI];  // per-lane byte offsets inside the wave's 16 rows
+  bool off_pool = false;
+  auto set_offsets = [&](uint32_t k_st, uint32_t v_st) {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int row = RPI * i + lane / CPR;
-    const int chunk = (lane % CPR) ^ swz<D>(row);
-    koff[i] = (uint32_t)(row * p.k_st + chunk * 16);
-    voff[i] = (uint32_t)(row * p.v_st + chunk * 16);
-  }
-  // The same inside 16 pool rows of one block (K and V alike): swz is linear
-  // over XOR, so the lane's chunk of row RPI i + r is c0 ^ swz(RPI i).
-  const uint32_t pool_row = kPaged ? (uint32_t)(lane / CPR) * (uint32_t)p.s_slot : 0u;
-  const uint32_t pool_c0 = (uint32_t)(((lane % CPR) ^ swz<D>(lane / CPR)) << 4);
-  auto pool_off = [&](int i) {
-    return (pool_c0 ^ (uint32_t)(swz<D>(RPI * i) << 4)) + pool_row +
-           (uint32_t)(i * RPI) * (uint32_t)p.s_slot;
+    for (int i = 0; i < NI; ++i) {
+      const uint32_t row = RPI * i + ln / CPR;
+      const uint32_t chunk = (ln % CPR) ^ swz<D>(row);
+      koff[i] = row * k_st + chunk * 16;
+      voff[i] = row * v_st + chunk * 16;
+    }
   };
+  // k/v token strides (below 2^27 bytes: host check), opaque so that they stay
+  // in scalar registers.  With the bases formed from the arguments per tile the
+  // compiler reloaded those, and waited for them, on every tile of k/v rows;
+  // the cursor's pointers advance by them instead.  head_dim 128, us: 32 prompts
+  // 33.5 -> 31.9, 9 prompts 19.2 -> 17.3, 28 decoding sequences with 4 prompts
+  // 32.2 -> 30.7; head_dim 64, 32/8 heads, 32 prompts 32.9 -> 32.3.
+  uint32_t k_st = (uint32_t)p.k_st, v_st = (uint32_t)p.v_st;
+  asm volatile("" : "+s"(k_st), "+s"(v_st));
+  set_offsets(k_st, v_st);
   // FP8 pool: a wave's 16 code rows (unswizzled, CRPI rows an instruction).
   const uint32_t code_lane =
       kF8 ? (uint32_t)(lane / CCPR) * (uint32_t)p.s_slot + (uint32_t)(lane % CCPR) * 16u : 0u;
@@ -514,10 +532,16 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
     int t, end;           // next tile to request, the item's last + 1
     int prefix, kend;
     int h, s;
-    int64_t base;         // key j of k/v is row base + j
+    const char* kb;       // tile t's first row of this wave in k and v (a key's
+    const char* vb;       // row is q0 + key - prefix, or k0 + key without a pool)
     int row0;             // `rows` holds the pool rows of tiles [row0, row0 + 64)
   };
   Cursor cu;
+  auto advance = [&]() {
+    ++cu.t;
+    cu.kb += (uint64_t)k_st * kKeyTile;
+    cu.vb += (uint64_t)v_st * kKeyTile;
+  };
   int64_t rows = -1;
   uint2 pend = make_uint2(0u, 0u);  // raw block ids that `rows` takes next
   auto cursor_to = [&](const Item& it) {
@@ -527,7 +551,11 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
     cu.end = it.t1;
     cu.h = it.h;
     cu.s = it.s;
-    cu.base = kPaged ? (int64_t)it.q0 - cu.prefix : (int64_t)it.k0;
+    const int64_t row = (kPaged ? (int64_t)it.q0 - cu.prefix : (int64_t)it.k0) +
+                        (int64_t)it.t0 * kKeyTile + 16 * wave;
+    const ColdArgs ca = cold_args();
+    cu.kb = uniform_ptr(ca->k + row * ca->k_st + it.h * ca->k_sh);
+    cu.vb = uniform_ptr(ca->v + row * ca->v_st + it.h * ca->v_sh);
     cu.row0 = it.t0;
   };
   // ---- pool rows (block16) ----
@@ -541,7 +569,6 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   // read block 0.
   auto load_ids = [&](int s, int t0, int prefix) {
     const ColdArgs ca = cold_args();
-    pend = make_uint2(0u, 0u);
     const int tok = (t0 + lane) * kKeyTile + 16 * wave;
     const int col = (int)fast_div((uint32_t)tok, cold_div(ca->bs_div));
     if (tok < prefix && col < ca->table_width) {
@@ -550,6 +577,8 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       const int64_t e = ((int64_t)s * ca->t_sb + col) << i64;
       pend.x = w[e];
       pend.y = w[e + i64];
+    } else {
+      pend = make_uint2(0u, 0u);
     }
   };
   auto take_ids = [&](int t0) {  // the requested ids are those of the cursor's tiles from t0 on
@@ -567,16 +596,14 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   // What `rows` will need next: the item's following 64 tiles, or the next
   // item's first.
   auto request_ids = [&](bool has_next, const Item& nxt) {
-    if constexpr (!kPaged) return;
-    if (cu.end - cu.row0 > 64) {
-      if (cu.prefix > (cu.row0 + 64) * kKeyTile) load_ids(cu.s, cu.row0 + 64, cu.prefix);
-    } else if (has_next && prefix_of(nxt) > 0) {
-      load_ids(nxt.s, nxt.t0, prefix_of(nxt));
-    }
+    const bool more = cu.end - cu.row0 > 64;
+    const int t0 = more ? cu.row0 + 64 : nxt.t0;
+    const int prefix = more ? cu.prefix : (has_next ? prefix_of(nxt) : 0);
+    if (prefix > t0 * kKeyTile) load_ids(more ? cu.s : nxt.s, t0, prefix);
   };
 
   // How the cursor's tile is requested.
-  enum { kNone, kRows, kPool, kCodes };
+  enum { kNone, kRows, kCodes };
   struct Easy {
     int kind;
     const char* kb;  // the wave's first row
@@ -667,8 +694,9 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
           // An FP8 pool row is staged by the code copy and its conversion.
           if constexpr (!kF8) pool_at(j, braw[i], chunk * 16, ka[i], va_[i]);
         } else {
-          ka[i] = ca->k + (cu.base + j) * ca->k_st + cu.h * ca->k_sh + chunk * 16;
-          va_[i] = ca->v + (cu.base + j) * ca->v_st + cu.h * ca->v_sh + chunk * 16;
+          const uint32_t r = row - 16 * wave;
+          ka[i] = cu.kb + (r * k_st + chunk * 16);
+          va_[i] = cu.vb + (r * v_st + chunk * 16);
         }
       }
     }
@@ -700,10 +728,13 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
     e.kb = e.vb = nullptr;
     const int kb = cu.t * kKeyTile;
     if (kb >= cu.prefix && kb + kKeyTile <= cu.kend) {
-      const int64_t row = cu.base + kb + 16 * wave;
       e.kind = kRows;
-      e.kb = uniform_ptr(p.k + row * p.k_st + cu.h * p.k_sh);
-      e.vb = uniform_ptr(p.v + row * p.v_st + cu.h * p.v_sh);
+      if (kPaged && !kF8 && off_pool) {
+        set_offsets(k_st, v_st);
+        off_pool = false;
+      }
+      e.kb = cu.kb;
+      e.vb = cu.vb;
       return e;
     }
     int64_t row = -1;
@@ -712,7 +743,12 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       row = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(rows >> 32), l) << 32) |
                       (uint32_t)__builtin_amdgcn_readlane((int)rows, l));
       if (kb + kKeyTile <= min(cu.prefix, cu.kend) && row >= 0 && p.block16) {
-        e.kind = kF8 ? kCodes : kPool;
+        e.kind = kF8 ? kCodes : kRows;
+        if (!kF8 && !off_pool) {
+          const uint32_t slot = (uint32_t)cold_args()->s_slot;
+          set_offsets(slot, slot);
+          off_pool = true;
+        }
         e.kb = uniform_ptr(p.kp + row);
         e.vb = uniform_ptr(p.vp + row);
         return e;
@@ -725,13 +761,9 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
     if constexpr (kv_once) {
       dma16_nt(koff[i], e.kb, dst + i * 1024);
       dma16_nt(voff[i], e.vb, dst + TILE_B + i * 1024);
-    } else if (!kPaged || kF8 || e.kind == kRows) {
+    } else {
       dma16(koff[i], e.kb, dst + i * 1024);
       dma16(voff[i], e.vb, dst + TILE_B + i * 1024);
-    } else {
-      const uint32_t o = pool_off(i);
-      dma16(o, e.kb, dst + i * 1024);
-      dma16(o, e.vb, dst + TILE_B + i * 1024);
     }
   };
   auto easy_codes = [&](const Easy& e, int i) {
@@ -741,7 +773,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   };
   auto issue_now = [&](const Easy& e, int st) {  // all of an easy tile at once
     const uint32_t dst = lds_base + (uint32_t)(st * 2 * TILE_B + wave * NI * 1024);
-    if (e.kind == kRows || e.kind == kPool) {
+    if (e.kind == kRows) {
 #pragma unroll
       for (int i = 0; i < NI; ++i) easy_issue(e, i, dst);
     }
@@ -816,7 +848,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   const int kswz = swz<D>(r16);
   const int vswz = swz<D>(4 * g4 + (r16 >> 2));
 
-  Item cur, nxt;
+  Item cur, nxt = {};
   if (!next_item(cur)) return;
   cursor_to(cur);
   if (kPaged && cu.prefix > 0) {
@@ -825,7 +857,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
   }
   if (cu.t < cu.end) {
     issue_now(issue(0), 0);
-    ++cu.t;
+    advance();
   }
   load_q(cur);
   uint2 st_slot = load_slot(cur);
@@ -833,7 +865,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
 
   for (;;) {
     const bool has_next = next_item(nxt);
-    request_ids(has_next, nxt);
+    if constexpr (kPaged) request_ids(has_next, nxt);
 
     const int pos0 = cur.qb * BQ;
     const int nrows = (min(cur.ql, pos0 + BQ) - pos0) * G;  // MFMA rows of the block in use
@@ -1019,23 +1051,20 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       // spread over the S^T loop below: issued back to back, they stall the
       // wave on the vector memory queue for as long as the MFMAs of half a
       // tile take.  Other tiles are issued here.
-      bool req = true;
-      if (cu.t == cu.end) {
-        if (has_next) {
-          cursor_to(nxt);
-          if constexpr (kPaged) take_ids(nxt.t0);
-        }
-        req = has_next && cu.t < cu.end;
-      } else if (kPaged && cu.t - cu.row0 == 64) {
-        take_ids(cu.t);
-        request_ids(has_next, nxt);
+      const bool ends = cu.t == cu.end;
+      if (ends && has_next) cursor_to(nxt);
+      if constexpr (kPaged) {
+        const bool window = !ends && cu.t - cu.row0 == 64;
+        if (window || (ends && has_next)) take_ids(cu.t);
+        if (window) request_ids(has_next, nxt);
       }
+      const bool req = cu.t < cu.end;
       Easy e;
       e.kind = kNone;
       e.kb = e.vb = nullptr;
       if (req) {
         e = issue(stage ^ 1);
-        ++cu.t;
+        advance();
       }
       const uint32_t n_dst = lds_base + (uint32_t)((stage ^ 1) * 2 * TILE_B + wave * NI * 1024);
       const char* s_k = s_kv + stage * 2 * TILE_B;
@@ -1118,7 +1147,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
 #pragma unroll
             for (int tt = 0; tt < NA; ++tt)
               sacc[tt][kt] = M::mfma(ka[kt & 1][ds], qreg[tt][ds], sacc[tt][kt]);
-          if (kt % EVERY == 0 && (e.kind == kRows || e.kind == kPool)) {
+          if (kt % EVERY == 0 && e.kind == kRows) {
 #pragma unroll
             for (int j = 0; j < PAIRS; ++j) easy_issue(e, (kt / EVERY) * PAIRS + j, n_dst);
           }
@@ -1223,7 +1252,7 @@ __global__ __launch_bounds__(kVarlenThreads, 2) void varlen_attention_kernel(Var
       if constexpr (kPaged) take_ids(nxt.t0);
       if (cu.t < cu.end) {
         issue_now(issue(stage), stage);
-        ++cu.t;
+        advance();
       }
       load_q(nxt);
       st_slot = load_slot(nxt);
