@@ -114,3 +114,66 @@ def test_split_launch_without_a_pool(dev, hq, hkv, d, causal, lens):
                                max(lens), scale=d ** -0.5, causal=causal)
     ref = oracle.varlen_attention(q, k, v, cu, cu, d ** -0.5, causal)
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+@pytest.mark.parametrize("bs", [16, 8])
+@pytest.mark.parametrize("dim", [0, 1, 2], ids=["block", "slot", "head"])
+def test_pool_with_a_negative_stride(dev, monkeypatch, dim, bs, kv):
+    # The C ABI takes pool strides of either sign: the pool lies reversed along
+    # one dimension and is described from that dimension's last element.
+    gen = torch.Generator().manual_seed(10 * bs + dim)
+    hq, hkv, d, seqs = 16, 8, 128, [(700, 1), (130, 70), (0, 90), (33, 5)]
+    ql, kl = [n for _, n in seqs], [p + n for p, n in seqs]
+    need = [math.ceil(n / bs) for n in kl]
+    nb = sum(need) + 1
+    perm = torch.randperm(nb, generator=gen)
+    table = torch.full((len(seqs), max(need)), -1, dtype=torch.int32)
+    at = 0
+    for s, m in enumerate(need):
+        table[s, :m] = perm[at:at + m]
+        at += m
+    slots = torch.tensor([int(table[s, j // bs]) * bs + j % bs
+                          for s, (p, n) in enumerate(seqs) for j in range(p, p + n)],
+                         dtype=torch.int32)
+    ks, vs = (0.05, 0.08) if kv == "fp8" else (1.0, 1.0)
+    kp, vp = (torch.randn(nb, bs, hkv, d, generator=gen) for _ in range(2))
+    if kv == "fp8":
+        kp, vp = oracle.quantize_fp8(kp, ks), oracle.quantize_fp8(vp, vs)
+    else:
+        kp, vp = kp.to(torch.bfloat16), vp.to(torch.bfloat16)
+    q = torch.randn(sum(ql), hq, d, generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn(sum(ql), hkv, d, generator=gen).to(torch.bfloat16) for _ in range(2))
+    cu_q, cu_k = _cu(ql), _cu(kl)
+    as_bytes = torch.uint8 if kv == "fp8" else torch.int16
+    monkeypatch.setattr(ops, "_FAST_LOADED", True)
+    monkeypatch.setattr(ops, "_FAST", None)
+    real = N.lib()
+
+    class Reversed:
+        def __getattr__(self, fn):
+            return self.launch if fn == "va_varlen_attention" else getattr(real, fn)
+
+        def launch(self, args, stream):
+            pool = args._obj.pool
+            field = ("stride_block", "stride_slot", "stride_head")[dim]
+            step = getattr(pool, field) * (1 if kv == "fp8" else 2)
+            pool.k += ((nb, bs, hkv)[dim] - 1) * step
+            pool.v += ((nb, bs, hkv)[dim] - 1) * step
+            setattr(pool, field, -getattr(pool, field))
+            return real.va_varlen_attention(args, stream)
+
+    monkeypatch.setattr(N, "lib", Reversed)
+    print(f"dimension {dim} reversed, block {bs} {kv}", flush=True)
+    kd, vd = (p.view(as_bytes).flip(dim).view(p.dtype).to(dev) for p in (kp, vp))
+    out = ops.varlen_attention(q.to(dev), k.to(dev), v.to(dev), cu_q.to(dev), cu_k.to(dev),
+                               max(ql), max(kl), scale=d ** -0.5, causal=True, k_cache=kd,
+                               v_cache=vd, block_tables=table.to(dev), slot_mapping=slots.to(dev),
+                               k_scale=ks, v_scale=vs)
+    torch.cuda.synchronize()
+    ref = oracle.varlen_attention(q, k, v, cu_q, cu_k, d ** -0.5, True, k_cache=kp, v_cache=vp,
+                                  block_tables=table, k_scale=ks, v_scale=vs)
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+    ek, ev = oracle.store_kvcache(k, v, kp, vp, slots, k_scale=ks, v_scale=vs)
+    assert torch.equal(kd.cpu().view(as_bytes).flip(dim), ek.view(as_bytes))
+    assert torch.equal(vd.cpu().view(as_bytes).flip(dim), ev.view(as_bytes))

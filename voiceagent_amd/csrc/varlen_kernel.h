@@ -181,6 +181,9 @@ __device__ inline int wave_scan(int x) {
 // of the visible keys or unmapped, so every tile takes the same number of
 // DMA instructions (the pipeline's vmcnt waits count them).
 __device__ __align__(16) const uint4 kZeroRow = {0u, 0u, 0u, 0u};
+// Pool byte offset of a row that is not there.  Any other value is an offset:
+// pool strides may be negative.
+constexpr int64_t kNoRow = INT64_MIN;
 
 // LDS layout of a staged K or V tile: kKeyTile rows of 2 D bytes, unpadded;
 // the 16-byte chunk c of row r sits at chunk position c ^ swz(r).  The XOR
@@ -542,7 +545,7 @@ varlen_attention_kernel(VarlenParams p) {
     cu.kb += (uint64_t)k_st * kKeyTile;
     cu.vb += (uint64_t)v_st * kKeyTile;
   };
-  int64_t rows = -1;
+  int64_t rows = kNoRow;
   uint2 pend = make_uint2(0u, 0u);  // raw block ids that `rows` takes next
   auto cursor_to = [&](const Item& it) {
     cu.t = it.t0;
@@ -560,7 +563,7 @@ varlen_attention_kernel(VarlenParams p) {
   };
   // ---- pool rows (block16) ----
   // Lane l of `rows` holds the pool byte offset of the wave's 16 rows of tile
-  // row0 + l (-1: a block id outside the pool).  Block ids are requested 64
+  // row0 + l (kNoRow: a block id outside the pool).  Block ids are requested 64
   // tiles at a time and a tile ahead of their use, so no tile waits for them
   // (looked up as the tile was requested, each pool tile cost a second
   // dependent round trip: 4 prompts of 200-300 tokens over prefixes of 2K-8K
@@ -588,7 +591,7 @@ varlen_attention_kernel(VarlenParams p) {
     const int64_t bid = ca->table_i64 ? (int64_t)(((uint64_t)pend.y << 32) | pend.x)
                                       : (int64_t)(int32_t)pend.x;
     const uint32_t tok = (uint32_t)((t0 + lane) * kKeyTile + 16 * wave);
-    rows = -1;
+    rows = kNoRow;
     if (bid >= 0 && bid < ca->num_blocks)
       rows = bid * ca->s_blk + (int64_t)fast_mod(tok, cold_div(ca->bs_div)) * ca->s_slot +
              cu.h * ca->s_head;
@@ -629,16 +632,16 @@ varlen_attention_kernel(VarlenParams p) {
     auto pool_at = [&](int j, const uint2& raw, int c16, const char*& ka, const char*& va_) {
       int64_t off = row;
       if (ca->block16) {
-        if (off >= 0) off += (j & 15) * ca->s_slot + c16;
+        if (off != kNoRow) off += (j & 15) * ca->s_slot + c16;
       } else {
         const int64_t bid = ca->table_i64 ? (int64_t)(((uint64_t)raw.y << 32) | raw.x)
                                           : (int64_t)(int32_t)raw.x;
-        off = -1;
+        off = kNoRow;
         if (bid >= 0 && bid < ca->num_blocks)
           off = bid * ca->s_blk + (int64_t)fast_mod((uint32_t)j, bs_div) * ca->s_slot +
                 cu.h * ca->s_head + c16;
       }
-      if (off >= 0) {
+      if (off != kNoRow) {
         ka = ca->kp + off;
         va_ = ca->vp + off;
       }
@@ -737,12 +740,12 @@ varlen_attention_kernel(VarlenParams p) {
       e.vb = cu.vb;
       return e;
     }
-    int64_t row = -1;
+    int64_t row = kNoRow;
     if (kPaged && kb < cu.prefix) {
       const int l = cu.t - cu.row0;
       row = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(rows >> 32), l) << 32) |
                       (uint32_t)__builtin_amdgcn_readlane((int)rows, l));
-      if (kb + kKeyTile <= min(cu.prefix, cu.kend) && row >= 0 && p.block16) {
+      if (kb + kKeyTile <= min(cu.prefix, cu.kend) && row != kNoRow && p.block16) {
         e.kind = kF8 ? kCodes : kRows;
         if (!kF8 && !off_pool) {
           const uint32_t slot = (uint32_t)cold_args()->s_slot;
@@ -1074,12 +1077,12 @@ varlen_attention_kernel(VarlenParams p) {
       // The rows go out non-temporally: nothing in the launch reads them back
       // (config 3: 40.4 -> 39.6 us per launch).
       if (fused_store && st_key0 < kb + kKeyTile && st_key0 + nrows / G > kb) {
-        // Pool offset of this lane's row (-1: not stored), computed in the
+        // Pool offset of this lane's row (kNoRow: not stored), computed in the
         // lane that holds the slot and handed to the lanes that store it.
         const int64_t cap = (int64_t)p.num_blocks * p.block_size;
         const int64_t slot = p.slot_i64 ? (int64_t)(((uint64_t)st_slot.y << 32) | st_slot.x)
                                           : (int64_t)(int32_t)st_slot.x;
-        int64_t at = -1;
+        int64_t at = kNoRow;
         if (slot >= 0 && slot < cap) {
           const int64_t blk = p.slot_small
                                   ? (int64_t)fast_div((uint32_t)slot, p.bs_div)
@@ -1094,7 +1097,7 @@ varlen_attention_kernel(VarlenParams p) {
           const int hi = __shfl((int)(at >> 32), holder, 64);
           const int row = st_base(k) + lane / CPR;
           const int key = st_key0 + row;
-          if (row < BQ && hi >= 0 && key >= kb && key < kb + kKeyTile) {
+          if (row < BQ && hi != (int)(kNoRow >> 32) && key >= kb && key < kb + kKeyTile) {
             const int64_t dst = (int64_t)(((uint64_t)(uint32_t)hi << 32) | lo) + c * 16;
             const int r = key - kb;
             const int off = r * ROWB + ((c ^ swz<D>(r)) << 4);
