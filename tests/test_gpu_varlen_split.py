@@ -177,3 +177,21 @@ def test_pool_with_a_negative_stride(dev, monkeypatch, dim, bs, kv):
     ek, ev = oracle.store_kvcache(k, v, kp, vp, slots, k_scale=ks, v_scale=vs)
     assert torch.equal(kd.cpu().view(as_bytes).flip(dim), ek.view(as_bytes))
     assert torch.equal(vd.cpu().view(as_bytes).flip(dim), ev.view(as_bytes))
+
+
+def test_loose_max_seqlen_q(dev):
+    # max_seqlen_q is any bound of the lengths; the largest a launch takes is
+    # 65535 * 16 query blocks of 128 rows, also where items of 64 rows would do.
+    hq, hkv, d, lens = 16, 2, 128, [4, 1, 2]
+    gen = torch.Generator().manual_seed(5)
+    q = torch.randn(sum(lens), hq, d, generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn(sum(lens), hkv, d, generator=gen).to(torch.bfloat16) for _ in range(2))
+    cu = _cu(lens)
+    bound = 65535 * 16 * (128 * hkv // hq)
+    out = ops.varlen_attention(q.to(dev), k.to(dev), v.to(dev), cu.to(dev), cu.to(dev), bound,
+                               max(lens), scale=d ** -0.5, causal=True)
+    ref = oracle.varlen_attention(q, k, v, cu, cu, d ** -0.5, True)
+    assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
+    with pytest.raises(N.NativeError, match="max_seqlen_q"):
+        ops.varlen_attention(q.to(dev), k.to(dev), v.to(dev), cu.to(dev), cu.to(dev), bound + 1,
+                             max(lens), scale=d ** -0.5, causal=True)

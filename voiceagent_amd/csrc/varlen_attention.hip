@@ -30,6 +30,8 @@ extern "C" size_t va_varlen_workspace_bytes(const va_varlen_args* a) {
 
 namespace va {
 
+constexpr int64_t kMaxQBlocks = 65535 * 16;  // query blocks of a sequence
+
 // Workspace of a split launch: pieces' o, (m, l), heads and counts.
 struct SplitLayout {
   size_t o, ml, head, count, total;
@@ -45,15 +47,14 @@ static SplitLayout split_layout(int head_dim) {
   return l;
 }
 
-// Whether a launch may gain from splitting its items, from what the host
-// knows.  The longest item may take as many tiles as the longest prompt or
-// the block table holds (the lengths themselves are on the device); with
-// items of half that on average, a slot's share is the piece the device would
-// choose.  The longest item has to exceed it by a quarter and five tiles
-// (~10 us): the pieces' partials and the merge launch cost about half that.
-// (9 prompts of 60-594 tokens and 24 decoding sequences beside three prompts
-// of 530, which this leaves whole, lost 2.5-3.4 us to a merge launch with
-// nothing to merge.)
+// Whether a launch can list `nqb` query blocks of every (sequence, kv head):
+// list indices are 32-bit.
+static bool list_fits(const va_varlen_args* a, int64_t nqb) {
+  const int64_t npairs = (int64_t)a->num_seqs * a->num_kv_heads;
+  return nqb <= kMaxQBlocks && npairs <= INT32_MAX / 2 &&
+         (npairs + kXcds - 1) / kXcds * nqb * kXcds <= INT32_MAX;
+}
+
 // Per XCD: slots, the items with `rows` MFMA rows each, and the tiles of the
 // longest item.
 struct VarlenLoad {
@@ -78,6 +79,15 @@ static int64_t split_piece(const VarlenLoad& w) {
   return std::max<int64_t>(w.items * w.longest / 2 / over, kSplitMinTiles);
 }
 
+// Whether a launch may gain from splitting its items, from what the host
+// knows.  The longest item may take as many tiles as the longest prompt or
+// the block table holds (the lengths themselves are on the device); with
+// items of half that on average, a slot's share is the piece the device would
+// choose.  The longest item has to exceed it by a quarter and five tiles
+// (~10 us): the pieces' partials and the merge launch cost about half that.
+// (9 prompts of 60-594 tokens and 24 decoding sequences beside three prompts
+// of 530, which this leaves whole, lost 2.5-3.4 us to a merge launch with
+// nothing to merge.)
 static bool split_wanted(const va_varlen_args* a) {
   if (a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0) return false;
   const int G = a->num_heads / a->num_kv_heads;
@@ -103,8 +113,12 @@ static bool split_wanted(const va_varlen_args* a) {
 // 24.5 / 23.4; 26 decoding sequences with 3 short prompts 21.3 / 18.7; chunks
 // of a few tokens over long prefixes 61.8 / 40.7; 9 prompts of 60-594 tokens
 // 39.2 / 37.2; 16 prompts of 109-439 (three rounds of half items) 39.8 / 45.8.
+// Nor does one whose max_seqlen_q (any bound of the lengths) makes more query
+// blocks of half the rows than a launch takes.
 static bool half_rows_wanted(const va_varlen_args* a, bool split) {
   if (!a->causal || a->prologue != nullptr) return false;
+  const int BQ = kRowsPerWG / 2 * a->num_kv_heads / a->num_heads;
+  if (!list_fits(a, ((int64_t)a->max_seqlen_q + BQ - 1) / BQ)) return false;
   const VarlenLoad full = varlen_load(a, kRowsPerWG), half = varlen_load(a, kRowsPerWG / 2);
   auto tiles = [&](const VarlenLoad& w) {
     const int64_t share = (w.items * w.longest / 2 + w.slots - 1) / w.slots;
@@ -227,9 +241,11 @@ int va::varlen_native(const va_varlen_args* a, void* stream) {
                      split_wanted(a) && a->workspace_bytes >= split_layout(a->head_dim).total;
   const bool half = half_rows_wanted(a, split);
   const int BQ = (half ? kRowsPerWG / 2 : kRowsPerWG) / G;
-  const int nqb = (a->max_seqlen_q + BQ - 1) / BQ;
+  const int nqb = (int)(((int64_t)a->max_seqlen_q + BQ - 1) / BQ);
   if (nqb == 0) return VA_OK;
-  VA_CHECK_ARG(nqb <= 65535 * 16, "va_varlen_attention: max_seqlen_q too large");
+  VA_CHECK_ARG(nqb <= kMaxQBlocks, "va_varlen_attention: max_seqlen_q too large");
+  VA_CHECK_ARG(list_fits(a, nqb),
+               "va_varlen_attention: too many (sequence, kv head, query block) items");
 
   VarlenParams p;
   p.q = (const char*)a->q;
@@ -321,8 +337,6 @@ int va::varlen_native(const va_varlen_args* a, void* stream) {
   // Persistent 1-D grid over kXcds interleaved item lists; see the kernel.
   const int64_t npairs = (int64_t)a->num_seqs * a->num_kv_heads;
   const int64_t items_per_xcd = (npairs + kXcds - 1) / kXcds * nqb;
-  VA_CHECK_ARG(npairs <= INT32_MAX / 2 && items_per_xcd * kXcds <= INT32_MAX,
-               "va_varlen_attention: too many (sequence, kv head, query block) items");
   const hipStream_t st = (hipStream_t)stream;
   const bool ok =
       a->dtype == VA_BF16
