@@ -275,7 +275,9 @@ typedef struct va_varlen_args {
   int32_t num_heads, num_kv_heads, head_dim;
   /* max_seqlen_q sizes the launch's query blocks and must be at least every
    * q_len (as flash_attn_varlen_func requires): query rows past it are not
-   * computed.  max_seqlen_k is not read (key ranges come from cu_seqlens_k). */
+   * computed.  Key ranges come from cu_seqlens_k; max_seqlen_k, where it is
+   * at least max_seqlen_q, only tells the launch how long contexts may be (a
+   * pool's table may be wider), for its choice of items and their splitting. */
   int32_t max_seqlen_q, max_seqlen_k;
   int32_t causal;         /* 1: bottom-right aligned causal mask          */
   float scale;

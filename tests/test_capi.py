@@ -141,6 +141,31 @@ def test_varlen_needs_no_workspace_even_for_long_fp8_prefixes():
     assert lib.va_varlen_workspace_bytes(ctypes.byref(args)) == 0
 
 
+def _varlen_args(total_q, max_q, max_k, *, seqs, table_width, hq=16, hkv=8, d=128, causal=1):
+    args = N.new_args(N.VarlenArgs)
+    args.num_seqs, args.total_q, args.max_seqlen_q, args.max_seqlen_k = seqs, total_q, max_q, max_k
+    args.num_heads, args.num_kv_heads, args.head_dim, args.causal = hq, hkv, d, causal
+    if table_width:
+        args.pool.k = args.pool.v = args.block_tables = 1 << 20  # never dereferenced
+        args.pool.block_size, args.pool.num_blocks = 16, 1 << 16
+        args.table_width = table_width
+    return args
+
+
+def test_varlen_splitting_follows_the_contexts_not_the_tables_width():
+    size = N.lib().va_varlen_split_workspace_bytes
+    # Nine prompts of up to 594 tokens have nothing worth splitting, whether
+    # their table is as wide as they are long or as the model's maximum.
+    for width in (38, 2048):
+        assert size(ctypes.byref(_varlen_args(2900, 594, 594, seqs=9, table_width=width))) == 0
+    # One token of a context of 4000 has.  Below max_seqlen_q, max_seqlen_k is
+    # no bound of anything: the table's width counts.
+    for max_k in (0, 4000):
+        assert size(ctypes.byref(_varlen_args(60, 57, max_k, seqs=4, table_width=250))) > 0
+    assert size(ctypes.byref(_varlen_args(60, 57, 60, seqs=4, table_width=250))) == 0
+    assert size(ctypes.byref(_varlen_args(60, 57, 4000, seqs=4, table_width=4))) == 0
+
+
 def test_ops_refuse_cpu_tensors():
     q = torch.zeros(2, 16, 128)
     pool = torch.zeros(4, 16, 8, 128)

@@ -56,15 +56,18 @@ static bool list_fits(const va_varlen_args* a, int64_t nqb) {
 }
 
 // Per XCD: slots, the items with `rows` MFMA rows each, and the tiles of the
-// longest item.
+// longest item.  Without the lengths, which are on the device, an item over a
+// pool may be as long as the block table is wide; max_seqlen_k, where it is a
+// bound at all, says less (an eager step's table may be the model's whole
+// width).  The lengths alone decide what is computed.
 struct VarlenLoad {
   int64_t slots, items, longest;
 };
 static VarlenLoad varlen_load(const va_varlen_args* a, int rows) {
   const int BQ = rows * a->num_kv_heads / a->num_heads;
-  const int64_t table_keys =
-      a->pool.k != nullptr ? (int64_t)a->table_width * a->pool.block_size : 0;
-  const int64_t keys = a->max_seqlen_q > table_keys ? a->max_seqlen_q : table_keys;
+  int64_t keys = a->pool.k != nullptr ? (int64_t)a->table_width * a->pool.block_size : 0;
+  if (a->max_seqlen_k >= a->max_seqlen_q) keys = std::min<int64_t>(keys, a->max_seqlen_k);
+  keys = std::max<int64_t>(keys, a->max_seqlen_q);
   VarlenLoad w;
   w.slots = 2 * (int64_t)current_device_cus() / kXcds;
   w.items = (a->num_kv_heads * ((int64_t)a->total_q / BQ + a->num_seqs) + kXcds - 1) / kXcds;
@@ -80,9 +83,7 @@ static int64_t split_piece(const VarlenLoad& w) {
 }
 
 // Whether a launch may gain from splitting its items, from what the host
-// knows.  The longest item may take as many tiles as the longest prompt or
-// the block table holds (the lengths themselves are on the device); with
-// items of half that on average, a slot's share is the piece the device would
+// knows.  With items of half the longest one's tiles on average, a slot's share is the piece the device would
 // choose.  The longest item has to exceed it by a quarter and five tiles
 // (~10 us): the pieces' partials and the merge launch cost about half that.
 // (9 prompts of 60-594 tokens and 24 decoding sequences beside three prompts

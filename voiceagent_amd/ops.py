@@ -656,8 +656,9 @@ def varlen_attention(
     ``k``/``v`` rows aligned with the queries (all from the pool if ``k`` is
     None).  ``slot_mapping`` fuses store_kvcache of k/v into the same launch.
     ``max_seqlen_q`` must be at least every q_len, as for flash-attn: it sizes
-    the launch, and query rows past it are not computed.  ``max_seqlen_k`` is
-    not read: key ranges come from ``cu_seqlens_k``.  An FP8 pool
+    the launch, and query rows past it are not computed.  Key ranges come from
+    ``cu_seqlens_k``; ``max_seqlen_k`` only bounds the context lengths for the
+    launch's choice of items (the block table may be wider).  An FP8 pool
     (float8_e4m3fn codes, values code * k_scale / v_scale) is converted tile
     by tile inside the kernel (no workspace); its new rows are stored
     quantised after the attention.  With a ``prologue`` (causal, head_dim
