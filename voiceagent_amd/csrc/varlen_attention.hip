@@ -82,13 +82,20 @@ static int64_t split_piece(const VarlenLoad& w) {
   return std::max<int64_t>(w.items * w.longest / 2 / over, kSplitMinTiles);
 }
 
-// Whether a launch may gain from splitting its items, from what the host
-// knows.  With items of half the longest one's tiles on average, a slot's share is the piece the device would
-// choose.  The longest item has to exceed it by a quarter and five tiles
-// (~10 us): the pieces' partials and the merge launch cost about half that.
-// (9 prompts of 60-594 tokens and 24 decoding sequences beside three prompts
-// of 530, which this leaves whole, lost 2.5-3.4 us to a merge launch with
-// nothing to merge.)
+// Whether a launch gains from splitting its items, from what the host knows.
+// With items of half the longest one's tiles on average, a slot's share is the
+// piece the device would choose.  The pieces' partials and the merge launch
+// cost 5-10 us, growing with the items, and a tile saved gives 1.2-1.5 us, so
+// over a prefix the longest item has to exceed a piece by a quarter and three
+// tiles and one more for each item of an XCD, up to nine.  Whole against
+// split, us, 16/8 heads of 128: 30 tokens over 400 keys 15.2 / 14.6; four such
+// prompts 15.8 / 17.1, at 64/8 heads 16.0 / 21.5; 64 over 1000 28.1 / 20.2.
+// New prompts' own blocks fill the slots with items whose lengths fall evenly,
+// which leaves splitting less to even out: one prompt of 420 tokens 15.3 /
+// 18.5, of 2500 (2.86 pieces long) 59.4 / 62.1, four of 300 15.5 / 20.5, and
+// at head_dim 64, 32/8 heads, 14.3 / 19.3.  It pays at 2.94 pieces and above
+// (8/8 heads of 128: 3000 tokens beside eight prompts of 100 62.4 / 55.3, one
+// of 4000 81.9 / 73.8), not for short ones (one of 1000 at 16/8 26.7 / 30.3).
 static bool split_wanted(const va_varlen_args* a) {
   if (a->num_kv_heads <= 0 || a->num_heads % a->num_kv_heads != 0) return false;
   const int G = a->num_heads / a->num_kv_heads;
@@ -100,7 +107,10 @@ static bool split_wanted(const va_varlen_args* a) {
   if ((pairs + kXcds - 1) / kXcds > 64) return false;  // the plan holds a pair per lane
   const VarlenLoad w = varlen_load(a, kRowsPerWG);
   const int64_t piece = split_piece(w);
-  return w.longest >= piece + piece / 4 + 5;
+  const int64_t prompt = ((int64_t)a->max_seqlen_q + kKeyTile - 1) / kKeyTile;
+  if (w.longest > prompt)  // over a prefix
+    return w.longest >= piece + piece / 4 + std::min<int64_t>(3 + w.items, 9);
+  return w.longest >= 32 && 10 * w.longest >= 29 * piece;
 }
 
 // Whether a causal launch takes items of 64 rows (kHalf).  The last slot to
