@@ -166,6 +166,18 @@ def test_varlen_splitting_follows_the_contexts_not_the_tables_width():
     assert size(ctypes.byref(_varlen_args(60, 57, 4000, seqs=4, table_width=4))) == 0
 
 
+def test_varlen_split_workspace_follows_the_launch():
+    size = N.lib().va_varlen_split_workspace_bytes
+    # Partials of at most 8 x 103 pieces of 128 rows (512 + 8 bytes a row at
+    # head_dim 128); a launch of few or short items takes what these can make.
+    most = 8 * 103 * (128 * 520 + 16) + 256
+    sizes = [size(ctypes.byref(_varlen_args(total, q, k, seqs=seqs, table_width=k // 16 + 1)))
+             for total, q, k, seqs in [(30, 30, 430, 1), (64, 64, 1064, 1), (1000, 300, 8192, 4),
+                                       (32, 1, 16000, 32)]]
+    assert 0 < sizes[0] < sizes[1] < sizes[2] <= most and 0 < sizes[3] <= most
+    assert sizes[0] < 4 << 20 and sizes[1] < 16 << 20
+
+
 def test_ops_refuse_cpu_tensors():
     q = torch.zeros(2, 16, 128)
     pool = torch.zeros(4, 16, 8, 128)

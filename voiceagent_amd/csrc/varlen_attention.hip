@@ -32,21 +32,6 @@ namespace va {
 
 constexpr int64_t kMaxQBlocks = 65535 * 16;  // query blocks of a sequence
 
-// Workspace of a split launch: pieces' o, (m, l), heads and counts.
-struct SplitLayout {
-  size_t o, ml, head, count, total;
-};
-static SplitLayout split_layout(int head_dim) {
-  const size_t pieces = (size_t)kXcds * kSplitSlots;
-  SplitLayout l;
-  l.o = 0;
-  l.ml = l.o + pieces * kRowsPerWG * head_dim * sizeof(float);
-  l.head = l.ml + pieces * kRowsPerWG * sizeof(float2);
-  l.count = l.head + pieces * sizeof(int4);
-  l.total = l.count + 256;
-  return l;
-}
-
 // Whether a launch can list `nqb` query blocks of every (sequence, kv head):
 // list indices are 32-bit.
 static bool list_fits(const va_varlen_args* a, int64_t nqb) {
@@ -78,7 +63,7 @@ static VarlenLoad varlen_load(const va_varlen_args* a, int rows) {
 // Tiles of a piece the device would choose (plan_split).
 static int64_t split_piece(const VarlenLoad& w) {
   const int64_t over =
-      std::min<int64_t>(std::max(w.slots - w.items / 4, (w.slots + 1) / 2), kSplitSlots / 2);
+      std::min<int64_t>(std::max(w.slots - w.items / 4, (w.slots + 1) / 2), kSplitOver);
   return std::max<int64_t>(w.items * w.longest / 2 / over, kSplitMinTiles);
 }
 
@@ -138,12 +123,40 @@ static bool half_rows_wanted(const va_varlen_args* a, bool split) {
   return half.items <= 2 * half.slots && tiles(half) * 7 < tiles(full) * 10;
 }
 
+// Workspace of a split launch: pieces' o, (m, l), heads and counts, for the
+// slots its plan may spread over: what is left of those resident beside the
+// fewest items there can be, or the pieces that the most and longest items make
+// (a bound by the hints of varlen_load, so the plan is held to it).  At 128
+// pieces of 128 rows whatever the launch, each took 68 MB at head_dim 128: 30
+// tokens over 400 keys take 2.2, four prompts of 200-300 over 2K-8K 55.
+struct SplitLayout {
+  int over, slots;
+  size_t o, ml, head, count, total;
+};
+static SplitLayout split_layout(const va_varlen_args* a, bool half) {
+  const int rows = half ? kRowsPerWG / 2 : kRowsPerWG;
+  const VarlenLoad w = varlen_load(a, rows);
+  const int64_t resident = waves_per_simd(a->head_dim, half) * (int64_t)current_device_cus() / kXcds;
+  const int64_t fewest = w.items - (a->num_seqs * (int64_t)a->num_kv_heads + kXcds - 1) / kXcds;
+  SplitLayout l;
+  l.over = (int)std::min({std::max(resident - fewest / 4, (resident + 1) / 2),
+                          (w.items * (w.longest + 2) + 1) / kSplitMinTiles, (int64_t)kSplitOver});
+  l.slots = split_pieces(l.over);
+  const size_t pieces = (size_t)kXcds * l.slots;
+  l.o = 0;
+  l.ml = l.o + pieces * rows * a->head_dim * sizeof(float);
+  l.head = l.ml + pieces * rows * sizeof(float2);
+  l.count = l.head + pieces * sizeof(int4);
+  l.total = l.count + 256;
+  return l;
+}
+
 }  // namespace va
 
 extern "C" size_t va_varlen_split_workspace_bytes(const va_varlen_args* a) {
   using namespace va;
   if (a == nullptr || a->struct_size != sizeof(va_varlen_args)) return 0;
-  return split_wanted(a) ? split_layout(a->head_dim).total : 0;
+  return split_wanted(a) ? split_layout(a, half_rows_wanted(a, true)).total : 0;
 }
 
 extern "C" int va_varlen_attention(const va_varlen_args* a, void* stream) {
@@ -248,8 +261,9 @@ int va::varlen_native(const va_varlen_args* a, void* stream) {
               a->head_dim, G);
     return VA_ERR_UNSUPPORTED;
   }
-  const bool split = a->workspace != nullptr && (uintptr_t)a->workspace % 16 == 0 &&
-                     split_wanted(a) && a->workspace_bytes >= split_layout(a->head_dim).total;
+  const bool split =
+      a->workspace != nullptr && (uintptr_t)a->workspace % 16 == 0 && split_wanted(a) &&
+      a->workspace_bytes >= split_layout(a, half_rows_wanted(a, true)).total;
   const bool half = half_rows_wanted(a, split);
   const int BQ = (half ? kRowsPerWG / 2 : kRowsPerWG) / G;
   const int nqb = (int)(((int64_t)a->max_seqlen_q + BQ - 1) / BQ);
@@ -332,12 +346,15 @@ int va::varlen_native(const va_varlen_args* a, void* stream) {
 
   p.half = half;
   p.split = split;
+  p.split_over = p.split_slots = 0;
   p.part_o = nullptr;
   p.part_ml = nullptr;
   p.part_head = nullptr;
   p.part_count = nullptr;
   if (split) {
-    const SplitLayout l = split_layout(a->head_dim);
+    const SplitLayout l = split_layout(a, half);
+    p.split_over = l.over;
+    p.split_slots = l.slots;
     char* const ws = (char*)a->workspace;
     p.part_o = (float*)(ws + l.o);
     p.part_ml = (float2*)(ws + l.ml);

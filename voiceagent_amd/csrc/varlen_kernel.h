@@ -82,13 +82,16 @@ struct VarlenParams {
   int32_t slot_i64;
   int32_t num_qblocks;
   int32_t num_seqs, num_kv_heads;
+  int32_t split_over, split_slots;  // kSplit, below; here, in a line read at the start
+                                    // (in a later one the plan waited 1 us for it)
   FastDiv bs_div, hkv_div;  // block_size, num_kv_heads
   int32_t slot_small;       // num_blocks * block_size <= 2^31: slots divide in 32 bits
   int32_t block16;          // block_size % 16 == 0: 16 rows from a multiple of 16 share a block
   float k_scale, v_scale;   // FP8 pool: element = code * scale
   int32_t kv_f8;            // the pool holds e4m3 codes (strides in bytes of codes)
-  // Split items (kSplit; all null / 0 without a workspace): per XCD
-  // kSplitSlots pieces, their (m, l) and o, what they belong to, how many.
+  // Split items (kSplit; all null / 0 without a workspace): split_over, the most
+  // slots of an XCD a plan spreads over; per XCD split_slots pieces, their
+  // (m, l) and o, what they belong to, how many.
   int32_t split;  // host: take the kSplit instantiation
   int32_t half;   // host: take the kHalf instantiation
   float* part_o;
@@ -153,10 +156,11 @@ constexpr int kXcds = 8;
 // Lazy-rescale slack of the online softmax, in log2 units (p <= 2^kLazy).
 constexpr float kLazy = 8.0f;
 
-// Splitting: the most pieces of split items on one XCD (the plan needs at
-// most twice the slots it spreads over, and spreads over at most half this
-// number) and the fewest tiles a piece holds (see plan_split in the kernel).
-constexpr int kSplitSlots = 128;
+// Splitting: the most slots of an XCD a plan spreads over, its pieces of split
+// items at most (the reason: plan_split in the kernel), and the fewest tiles a
+// piece holds.
+constexpr int kSplitOver = 64;
+constexpr int split_pieces(int over) { return (8 * over + 4) / 5; }
 constexpr int kSplitMinTiles = 2;
 constexpr int kSplitMaxTiles = 1 << 18;  // longer contexts are not split (float division)
 
@@ -363,8 +367,8 @@ varlen_attention_kernel(VarlenParams p) {
   // of a piece; an item longer than that by a quarter is cut into equal
   // pieces of at most that many plus a quarter.  tile_sum is an upper bound
   // of the tiles (prefix tiles rounded up to quarters, one per item for the
-  // rest), so split items have at most 2 tile_sum / piece <= kSplitSlots
-  // pieces.
+  // rest), at most split_over pieces long, and an item of n >= 2 pieces is more
+  // than n - 3/4 pieces long: at most 8/5 split_over pieces in all.
   // (Stores of the plan's words are uniform, by all lanes of a wave: a branch
   // on the lane in this walk would make every value after it divergent, the
   // DMAs' scalar bases among them.)
@@ -384,7 +388,7 @@ varlen_attention_kernel(VarlenParams p) {
     if (__builtin_amdgcn_ballot_w64(nt >= kSplitMaxTiles || lnq > 1024 || sum >= (1 << 24)) != 0) return;
     const int tile_sum = __builtin_amdgcn_readlane(wave_scan(sum), 63);
     const int items = __builtin_amdgcn_readlane(wave_scan(lnq), 63);
-    const int over = min(max(nslots - items / 4, (nslots + 1) / 2), kSplitSlots / 2);
+    const int over = min(max(nslots - items / 4, (nslots + 1) / 2), p.split_over);
     const int pc = max(__builtin_amdgcn_readfirstlane((tile_sum + over - 1) / over), kSplitMinTiles);
     if (__builtin_amdgcn_ballot_w64(nt > pc + pc / 4) != 0) {
       piece = pc;
@@ -1273,7 +1277,7 @@ varlen_attention_kernel(VarlenParams p) {
     if (kSplit && cur.slot >= 0) {
       // A piece of a split item: unnormalised, in fp32, straight from the
       // accumulators (64-byte pieces of 16 rows an instruction).
-      const int64_t ps = (int64_t)xcd * kSplitSlots + cur.slot;
+      const int64_t ps = (int64_t)xcd * p.split_slots + cur.slot;
       if (wave == 0) p.part_head[ps] = make_int4(cur.npc, cur.q0 + pos0, nrows, cur.h);
 #pragma unroll
       for (int tt = 0; tt < NR; ++tt) {
@@ -1282,10 +1286,10 @@ varlen_attention_kernel(VarlenParams p) {
         lt = sum_xor16(lt);
         lt = sum_xor32(lt);
         if (row < nrows) {
-          float* const po = p.part_o + (ps * kRowsPerWG + row) * D + 4 * g4;
+          float* const po = p.part_o + (ps * (64 * NR) + row) * D + 4 * g4;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4_t*>(po + 16 * dt) = o[tt][dt];
-          if (g4 == 0) p.part_ml[ps * kRowsPerWG + row] = make_float2(m[tt], lt);
+          if (g4 == 0) p.part_ml[ps * (64 * NR) + row] = make_float2(m[tt], lt);
         }
       }
     } else if (cur.t0 < tend) {
@@ -1342,20 +1346,21 @@ varlen_attention_kernel(VarlenParams p) {
 // of the item whose first piece is XCD x % 8's piece x / 8 (the XCD that wrote
 // it), and ends at once when there is no such item.
 //   out = sum_j 2^(m_j - M) o_j / sum_j 2^(m_j - M) l_j,  M = max_j m_j.
-template <bool kBF16, int D, int G>
+template <bool kBF16, int D, int G, bool kHalf>
 __global__ __launch_bounds__(256) void varlen_merge_kernel(VarlenParams p) {
   constexpr int LPR = D / 4;       // lanes per row, four outputs each
   constexpr int RPP = 256 / LPR;   // rows per pass
+  constexpr int rows = kHalf ? kRowsPerWG / 2 : kRowsPerWG;  // of a piece's partials
   const int xcd = (int)blockIdx.x % kXcds, slot = (int)blockIdx.x / kXcds;
-  const int64_t ps = (int64_t)xcd * kSplitSlots + slot;
+  const int64_t ps = (int64_t)xcd * p.split_slots + slot;
   const int count = p.part_count[xcd];
   const int4 hd = p.part_head[ps];  // read whether or not it was written
   const int row0 = (int)blockIdx.y * 32;
   if (slot >= count || hd.x == 0 || row0 >= hd.z) return;
   const int col = threadIdx.x % LPR;
   for (int row = row0 + threadIdx.x / LPR; row < min(row0 + 32, hd.z); row += RPP) {
-    const float* po = p.part_o + (ps * kRowsPerWG + row) * D + 4 * col;
-    const float2* pm = p.part_ml + ps * kRowsPerWG + row;
+    const float* po = p.part_o + (ps * rows + row) * D + 4 * col;
+    const float2* pm = p.part_ml + ps * rows + row;
     float M = -1.0e30f, L = 0.f;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
     for (int j0 = 0; j0 < hd.x; j0 += 4) {
@@ -1363,7 +1368,7 @@ __global__ __launch_bounds__(256) void varlen_merge_kernel(VarlenParams p) {
       float2 ml[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int64_t at = min(j0 + j, hd.x - 1) * (int64_t)kRowsPerWG;
+        const int64_t at = min(j0 + j, hd.x - 1) * (int64_t)rows;
         ml[j] = pm[at];
         oj[j] = *reinterpret_cast<const f32x4_t*>(po + at * D);
       }
@@ -1414,8 +1419,8 @@ static void launch_grid(const VarlenParams& p, int64_t items_per_xcd, hipStream_
   if (per_xcd < 1) per_xcd = 1;
   hipLaunchKernelGGL(kern, dim3((unsigned)(per_xcd * kXcds)), dim3(kVarlenThreads), 0, st, p);
   if constexpr (kSplit)
-    hipLaunchKernelGGL((varlen_merge_kernel<kBF16, D, G>), dim3(kSplitSlots * kXcds, 4), dim3(256),
-                       0, st, p);
+    hipLaunchKernelGGL((varlen_merge_kernel<kBF16, D, G, kHalf>),
+                       dim3(p.split_slots * kXcds, kHalf ? 2 : 4), dim3(256), 0, st, p);
 }
 
 template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce = false,
