@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define VA_ATTN_ABI_VERSION 6
+#define VA_ATTN_ABI_VERSION 7
 
 /* status codes */
 #define VA_OK 0
@@ -296,8 +296,8 @@ typedef struct va_varlen_args {
   /* Optional (no varlen launch needs a workspace; va_varlen_workspace_bytes
    * returns 0): with at least va_varlen_split_workspace_bytes, 16-byte
    * aligned, the launch may split long items' keys over several workgroups.
-   * No initialisation needed; launches sharing one must be ordered on one
-   * stream.  An FP8 pool's prefix rows are converted to the 16-bit type
+   * No initialisation needed; it is written, so launches sharing one must be
+   * ordered on one stream (ABI 6 and earlier left the field unused).  An FP8 pool's prefix rows are converted to the 16-bit type
    * (code * scale, rounded once) inside the kernel, tile by tile, and its
    * new rows are stored quantised after the attention. */
   void* workspace;
@@ -324,9 +324,11 @@ size_t va_varlen_workspace_bytes(const va_varlen_args* args);
 
 /* Bytes of workspace with which va_varlen_attention may split these
  * arguments' long items over several workgroups (few items, or some with far
- * more keys than the others); 0 where splitting cannot help.  Without it the
- * launch gives the same result unsplit.  Depends on the current device's
- * compute-unit count. */
+ * more keys than the others); 0 where splitting does not help.  Without it, or
+ * with less, the launch runs unsplit.  A split launch sums in another order and
+ * rounds P to 16 bits against other reference maxima, so its result equals the
+ * unsplit one up to rounding, and in its last bits depends on the launch's
+ * other sequences.  Depends on the current device's compute-unit count. */
 size_t va_varlen_split_workspace_bytes(const va_varlen_args* args);
 
 /* ----------------------------------------------------------------- misc */
