@@ -707,6 +707,17 @@ varlen_attention_kernel(VarlenParams p) {
         }
       }
     }
+    // A lane that uses no block id leaves its load pending, and the compiler
+    // waits for it where the register is next written.  At head_dim 64 that was
+    // behind the DMA, on every tile: a partial tile, an item's last one, was
+    // waited for as soon as it was requested.  us, 32/8 heads: four prompts of
+    // 300 14.6 -> 13.9, 9 of 60-594 22.5 -> 21.4, 28 decoding sequences with 4
+    // prompts 20.6 -> 19.9; 64/8 heads, 32 of 50-450 69.7 -> 67.1.  (head_dim
+    // 128 has other registers there and no such wait.)
+    if constexpr (kPaged && !kF8 && D == 64) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) asm volatile("" ::"v"(braw[i].x), "v"(braw[i].y));
+    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       if constexpr (kv_once) {
