@@ -52,11 +52,14 @@ def test_tile_edges_over_nan_tails(dev, lens, exact, kv):
             p.view(torch.uint8)[~live] = 0x7F
         else:
             p[~live] = float("nan")
+    # Four contexts of 8192 would be cut over the CUs: whole, each of a
+    # workgroup's eight waves has 64 tiles and refills its window.
+    split = 8704 if len(lens) == 4 else ops.SPLIT_EXACT if exact else 0
     print(f"{len(lens)} contexts up to {max(lens)}, {kv}", flush=True)
     out = ops.paged_decode(q.to(dev), kp.to(dev), vp.to(dev), table.to(dev),
                            torch.tensor(lens, dtype=torch.int32, device=dev),
                            max_seq_len=max(lens) if exact else 32768, scale=D ** -0.5,
-                           split_tokens=ops.SPLIT_EXACT if exact else 0, k_scale=ks, v_scale=ks)
+                           split_tokens=split, k_scale=ks, v_scale=ks)
     assert (out.float().cpu() - ref).abs().max().item() <= 2e-2
 
 
