@@ -13,8 +13,9 @@
 // Tiling (one workgroup = 4 wave64 = 256 lanes): an item is one
 // (sequence, kv head, query block) with all G query heads of the kv group,
 // so its 128 MFMA rows are BQ = 128 / G query positions x G heads, row
-// r = position G + head: a short block fills the first rows only.  Wave w
-// owns the 16-row tiles w and w + 4 (items of 64 rows, kHalf: tile w).
+// r = position G + head: a short block's rows are the first ones, next to one
+// another.  Wave w owns the 16-row tiles w and w + 4 (items of 64 rows, kHalf:
+// tile w).
 // Workgroups are persistent: the grid fills the
 // GPU's workgroup slots once and each workgroup works through a list of
 // items.  Keys stream through LDS in 64-key tiles (K and V row-major,
@@ -1134,9 +1135,9 @@ varlen_attention_kernel(VarlenParams p) {
         }
       };
 
-      // One tile on the wave's first NA row tiles.
-      auto reduce = [&](auto NA_) {
-        constexpr int NA = decltype(NA_)::value;
+      // The tile, as a lambda: written in place, the kernels spill up to 17 more
+      // registers.
+      auto reduce = [&]() {
         // ---- S^T = K Q^T ----
         // K rows of 16-key group kt + 1 are read before group kt's DMA pair:
         // no LDS read moves across a DMA.
@@ -1147,7 +1148,7 @@ varlen_attention_kernel(VarlenParams p) {
         // bases: held through the loop they make the compiler spill.
         int k0 = (g4 ^ kswz) << 4, krow = r16 * ROWB;
         if constexpr (D > 64) asm volatile("" : "+v"(k0), "+v"(krow));
-        f32x4_t sacc[NA][KT];
+        f32x4_t sacc[NR][KT];
         uint4 ka[2][DS];
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) ka[0][ds] = lds_read16(s_k, krow + (k0 ^ (ds << 6)));
@@ -1159,11 +1160,11 @@ varlen_attention_kernel(VarlenParams p) {
               ka[(kt + 1) & 1][ds] = lds_read16(s_k, 16 * (kt + 1) * ROWB + krow + (k0 ^ (ds << 6)));
           }
 #pragma unroll
-          for (int tt = 0; tt < NA; ++tt) sacc[tt][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          for (int tt = 0; tt < NR; ++tt) sacc[tt][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int ds = 0; ds < DS; ++ds)
 #pragma unroll
-            for (int tt = 0; tt < NA; ++tt)
+            for (int tt = 0; tt < NR; ++tt)
               sacc[tt][kt] = M::mfma(ka[kt & 1][ds], qreg[tt][ds], sacc[tt][kt]);
           if (kt % EVERY == 0 && e.kind == kRows) {
 #pragma unroll
@@ -1197,9 +1198,9 @@ varlen_attention_kernel(VarlenParams p) {
         // which the fp32 sums and 16-bit P hold exactly as well.  Key masking
         // is applied only on tiles that cross a row's limit.
         const bool need_mask = kb + kKeyTile > lim_lo;
-        uint4 pb[NA][KS];
+        uint4 pb[NR][KS];
 #pragma unroll
-        for (int tt = 0; tt < NA; ++tt) {
+        for (int tt = 0; tt < NR; ++tt) {
           float sv[KT][4];
           if (need_mask) {
             const int rel = lim[tt] - kb - 4 * g4;  // key 16 kt + i of this lane is visible iff < rel
@@ -1254,12 +1255,12 @@ varlen_attention_kernel(VarlenParams p) {
           for (int dt = 0; dt < DT; ++dt) {
             const uint4 a = vf[dt % (DT / 4)];
 #pragma unroll
-            for (int tt = 0; tt < NA; ++tt) o[tt][dt] = M::mfma(a, pb[tt][ks], o[tt][dt]);
+            for (int tt = 0; tt < NR; ++tt) o[tt][dt] = M::mfma(a, pb[tt][ks], o[tt][dt]);
             const int nx = ks * DT + dt + DT / 4;
             if (nx < KS * DT) vf[dt % (DT / 4)] = read_v(nx / DT, nx % DT);
           }
       };
-      reduce(std::integral_constant<int, NR>{});
+      reduce();
       stage ^= 1;
     }
     if (cur.t0 == tend && has_next) {
@@ -1490,6 +1491,14 @@ static void launch_varlen(const VarlenParams& p, bool causal, int64_t items_per_
 template <bool kBF16, int D>
 bool launch_varlen_d(int G, const VarlenParams& p, bool causal, int64_t items_per_xcd,
                      hipStream_t st);
+template <>
+bool launch_varlen_d<true, 64>(int, const VarlenParams&, bool, int64_t, hipStream_t);
+template <>
+bool launch_varlen_d<true, 128>(int, const VarlenParams&, bool, int64_t, hipStream_t);
+template <>
+bool launch_varlen_d<false, 64>(int, const VarlenParams&, bool, int64_t, hipStream_t);
+template <>
+bool launch_varlen_d<false, 128>(int, const VarlenParams&, bool, int64_t, hipStream_t);
 
 template <bool kBF16, int D>
 static bool dispatch_varlen_g(int G, const VarlenParams& p, bool causal, int64_t items_per_xcd,
