@@ -44,7 +44,10 @@ static bool list_fits(const va_varlen_args* a, int64_t nqb) {
 // longest item.  Without the lengths, which are on the device, an item over a
 // pool may be as long as the block table is wide; max_seqlen_k, where it is a
 // bound at all, says less (an eager step's table may be the model's whole
-// width).  The lengths alone decide what is computed.
+// width).  The lengths alone decide what is computed.  Slots are counted two a
+// CU at head_dim 64 too, where three or four are resident: counted so, both
+// rules below took more than they should (64/8 heads of 64, one prompt of 1000
+// tokens 31.7 -> 40.3 us; 28 decoding sequences with 4 prompts 25.7 -> 33.6).
 struct VarlenLoad {
   int64_t slots, items, longest;
 };
@@ -100,15 +103,16 @@ static bool split_wanted(const va_varlen_args* a) {
 
 // Whether a causal launch takes items of 64 rows (kHalf).  The last slot to
 // end has about max(longest item, tiles / slots) tiles (a piece when split);
-// with 64 rows an item's tile takes 0.6-0.7 of the time, and there are up to
-// twice the items, whose set-up and staging cost more than that once they
+// with 64 rows an item's tile takes 0.8 of the time where it waits for nothing
+// else (580 more tokens in one prompt, nine tiles: 11.4 us against 13.8; 0.7 in
+// the rule), and there are up to twice the items, whose set-up and staging cost more than that once they
 // come in more than two rounds.  So short blocks (decoding sequences, chunks
 // of a few tokens) and launches that do not fill the slots take them; a full
 // launch of prompts, or long prefixes over enough rows to fill the slots, do
-// not.  128 against 64 rows, us with the prologue: one prompt of 420 tokens
-// 24.5 / 23.4; 26 decoding sequences with 3 short prompts 21.3 / 18.7; chunks
-// of a few tokens over long prefixes 61.8 / 40.7; 9 prompts of 60-594 tokens
-// 39.2 / 37.2; 16 prompts of 109-439 (three rounds of half items) 39.8 / 45.8.
+// not.  128 against 64 rows, us, 16/8 heads of 128: one prompt of 420 tokens
+// 18.1 / 15.3; 28 decoding sequences with 4 prompts 29.0 / 25.6; 8 chunks of a
+// few tokens over 1K-4K, split, 41.4 / 39.9; 9 prompts of 60-594 tokens 24.1 /
+// 22.5; 16 of 109-439 (three rounds of half items) 24.5 / 27.3.
 // Nor does one whose max_seqlen_q (any bound of the lengths) makes more query
 // blocks of half the rows than a launch takes.
 static bool half_rows_wanted(const va_varlen_args* a, bool split) {

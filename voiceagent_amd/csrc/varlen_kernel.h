@@ -237,8 +237,8 @@ constexpr int waves_per_simd(int d, bool half) { return d == 64 ? (half ? 4 : 3)
 // a launch of 32 prompts).
 //
 // kHalf: 64 MFMA rows per item, one 16-row tile per wave.  A tile's body is
-// bound by the wave's own chain (S^T, softmax, O^T; ~2 us with two row tiles,
-// ~1.2 with one, alone on a CU), so a launch that leaves slots idle, or whose
+// bound by the wave's own chain (S^T, softmax, O^T; ~1.5 us with two row tiles,
+// ~1.25 with one, alone on a CU), so a launch that leaves slots idle, or whose
 // blocks are short anyway, ends sooner on items of half the rows (the host's
 // rule: half_rows_wanted).
 template <bool kBF16, int D, int G, bool kCausal, bool kPaged, bool kOnce, bool kF8, bool kPro,

@@ -26,10 +26,11 @@ store-then-attend order with two launches.
 the rotary cos/sin cache and the tokens' positions): q and k are then the
 raw projections, and the layer applies RMSNorm and RoPE to them as
 Qwen3Attention.forward does before calling attention (models/qwen3.py:42-48).
-A decode batch with the fused store applies it inside the decode launch.  A
-prefill batch (head_dim 128, 16-bit pool or none) runs ``ops.qk_norm_rope``
-over the keys alone and lets the varlen launch normalise and rotate the
-queries itself; any other batch runs ``ops.qk_norm_rope`` over both first.
+A decode batch with the fused store applies it inside the decode launch; any
+other batch runs ``ops.qk_norm_rope`` over both first.  (With
+``varlen_fuse_prologue`` a prefill batch, at head_dim 128 over a 16-bit pool or
+none, runs it over the keys alone and lets the varlen launch normalise and
+rotate the queries.)
 Qwen3Attention then passes the prologue instead of calling q_norm, k_norm and
 rotary_emb itself.
 
@@ -94,12 +95,12 @@ def _decode_split(context) -> int:
 class PagedAttention(nn.Module):
     fuse_store = True
     # True: prefill batches let the varlen launch apply the query prologue
-    # (the keys alone go through the standalone kernel first).  Off by
-    # default: over config 3 both ways take 66 us per layer, as each item
-    # of the varlen launch fetches the cos / sin rows of its 64 positions
-    # for one KV head (8 times the standalone kernel's rotary traffic per
-    # position), which costs what the saved query round trip through HBM
-    # saves.  False: the standalone kernel over q and k, then the launch.
+    # (the keys alone go through the standalone kernel first).  False: the
+    # standalone kernel over q and k, then the launch.  Which is faster depends
+    # on the batch: 32 prompts of 50-450 tokens take 55.6 us fused and 61.9 in
+    # two launches (28 input sets), but a fused launch does not take items of 64 rows, which
+    # small batches want (one prompt of 420 tokens 26.3 against 22.5, 28
+    # decoding sequences with 4 prompts 37 against 30).  Off by default.
     varlen_fuse_prologue = False
     kv_layout = ops.LAYOUT_NHD
     k_scale = 1.0  # FP8 pools: value of a key code = code * k_scale

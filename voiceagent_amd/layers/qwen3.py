@@ -13,7 +13,7 @@ model runner binds its cache slices the same way
   store_kvcache and attention as separate launches).
 * Other batches run the standalone prologue kernel over q and k, then the
   varlen path of :class:`PagedAttention`.  With ``varlen_fuse_prologue``
-  set (off by default: no faster over config 3), prefill batches with
+  set (off by default: faster for large prompt batches alone), prefill batches with
   head_dim 128 and a 16-bit pool or none run the standalone kernel over the
   keys alone, and the varlen launch normalises and rotates the queries
   itself, in registers, at each item's first key tile.
