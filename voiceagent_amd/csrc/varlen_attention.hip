@@ -105,14 +105,17 @@ static bool split_wanted(const va_varlen_args* a) {
 // end has about max(longest item, tiles / slots) tiles (a piece when split);
 // with 64 rows an item's tile takes 0.8 of the time where it waits for nothing
 // else (580 more tokens in one prompt, nine tiles: 11.4 us against 13.8; 0.7 in
-// the rule), and there are up to twice the items, whose set-up and staging cost more than that once they
-// come in more than two rounds.  So short blocks (decoding sequences, chunks
-// of a few tokens) and launches that do not fill the slots take them; a full
-// launch of prompts, or long prefixes over enough rows to fill the slots, do
-// not.  128 against 64 rows, us, 16/8 heads of 128: one prompt of 420 tokens
+// the rule), and there are up to twice the items, whose set-up and staging
+// cost more than that once they come in more than two rounds (one and a half
+// at group 8, where a tile is staged for eight positions).  So short blocks
+// (decoding sequences, chunks of a few tokens) and launches that do not fill
+// the slots take them; a full launch of prompts, or long prefixes over enough
+// rows to fill the slots, do not.  128 against 64 rows, us, 16/8 heads of 128: one prompt of 420 tokens
 // 18.1 / 15.3; 28 decoding sequences with 4 prompts 29.0 / 25.6; 8 chunks of a
 // few tokens over 1K-4K, split, 41.4 / 39.9; 9 prompts of 60-594 tokens 24.1 /
-// 22.5; 16 of 109-439 (three rounds of half items) 24.5 / 27.3.
+// 22.5; 16 of 109-439 (three rounds of half items) 24.5 / 27.3; 64/8 heads:
+// one of 700 (88 items) 28.1 / 27.1, one of 1000 (126) 38.2 / 43.0, two of 500
+// 24.7 / 27.8.
 // Nor does one whose max_seqlen_q (any bound of the lengths) makes more query
 // blocks of half the rows than a launch takes.
 static bool half_rows_wanted(const va_varlen_args* a, bool split) {
@@ -124,7 +127,8 @@ static bool half_rows_wanted(const va_varlen_args* a, bool split) {
     const int64_t share = (w.items * w.longest / 2 + w.slots - 1) / w.slots;
     return std::max(split ? split_piece(w) : w.longest, share);
   };
-  return half.items <= 2 * half.slots && tiles(half) * 7 < tiles(full) * 10;
+  const int64_t most = a->num_heads == 8 * a->num_kv_heads ? half.slots * 3 / 2 : 2 * half.slots;
+  return half.items <= most && tiles(half) * 7 < tiles(full) * 10;
 }
 
 // Workspace of a split launch: pieces' o, (m, l), heads and counts, for the
@@ -132,7 +136,7 @@ static bool half_rows_wanted(const va_varlen_args* a, bool split) {
 // fewest items there can be, or the pieces that the most and longest items make
 // (a bound by the hints of varlen_load, so the plan is held to it).  At 128
 // pieces of 128 rows whatever the launch, each took 68 MB at head_dim 128: 30
-// tokens over 400 keys take 2.2, four prompts of 200-300 over 2K-8K 55.
+// tokens over 400 keys take 2.1, four prompts of 200-300 over 2K-8K 52.
 struct SplitLayout {
   int over, slots;
   size_t o, ml, head, count, total;
